@@ -1,6 +1,6 @@
 // The two consumers of the in-projection output that forward_gtree calls by default: the full-attention prep and
-// the linear-attention prep on the tree layout. Both are one workgroup per token row: the row is read once,
-// finished in LDS, and written out with whole 8- or 16-byte vector stores.
+// the linear-attention prep on the tree layout. Both give every wave a piece of a token row that it reads, finishes
+// and writes out by itself, with whole 8- or 16-byte vector stores.
 #include "ojx_internal.h"
 
 namespace ojx {
@@ -127,142 +127,141 @@ hipError_t launch_fullattn_prep(const uint16_t* proj, int64_t N, int HQ, int HKV
 // Products of two bf16 values are exact in fp32, so the conv's sum order is the only one that fixes its bits; it is
 // kept. The head sums of squares are added in another order than the reference's (one rounding step at most).
 //
-// Work layout: one workgroup of 8 waves (kLinThreads = 512 lanes) per packed row, grid = N rows + the padding
-// groups.
-//   1. conv + SiLU for all C channels (8 per lane per step, the four history rows and the 64 weight bytes as 16-byte
-//      loads; 10240 channels take 2.5 steps), the bf16 results kept in an LDS copy of the row;
-//   2. one q/k head per wave at a time, 2 channels per lane: wave-total sum of squares, scaled in place in LDS;
-//      lanes below HV compute the gates into LDS meanwhile;
-//   3. the finished row is written slot after slot: every 16-byte chunk of a slot's q | k | v row is one lane's
-//      LDS read and global store, so each slot row goes out as one contiguous sweep; slot ids come in through
-//      LDS, kLinThreads at a time (the first batch fetched before step 1).
-// A padding group (the workgroups after the N row workgroups) writes zero rows to kPadSlots consecutive
-// padding slots.
-constexpr int kPadSlots = 8;
+// Work layout: one wave per (row, 512 channels), eight consecutive channels per lane; four consecutive rows of one
+// channel block per workgroup, so that the block's weights and the rows' shared history come from L1 after the first
+// wave. A lane keeps its finished channels as one 16-byte value in registers and stores it to every slot of the row:
+// 1 KB contiguous per wave and slot, slot ids fetched 64 at a time beside the row's loads and read lane by lane (a
+// uniform address per store). A head of 128 channels is 16 lanes, so its sum of squares is four shuffles. No LDS and
+// no barrier: the waves are independent, where an earlier kernel of one workgroup per row (about one workgroup per CU
+// on a 288-row tree) exposed every latency of its conv -> barrier -> norm -> barrier -> write chain. One more channel
+// block, the last, computes the gates. The row groups after the rows write zeros to the padding slots, kPadGroups
+// slots at a time.
+// What bounds it: the slot rows written, once a tree has a few hundred slots (below that, the launch and one chain of
+// loads). The slot stores are non-temporal: every line is written whole and read by another kernel, and the hint took
+// the largest tree below from 118.4 to 85-98 us (the channel blocks of a row are neighbouring workgroups, so that its
+// 20 KB of each slot go out at about the same time). Graph replays on MI355X, earlier kernel -> this one, and the
+// algorithmic rate: 200 shared rows x 8 paths 16.3 -> 9.8 us (4.4 TB/s), 480 x 8 25.8 -> 18.4, 40 x 4 9.8 -> 4.6,
+// 1600 x 3 42.0 -> 30.4, 1500 x 16 124.4 -> 85-98 us (5.5-6.4 TB/s; a fill reaches 6.9).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store_nt(uint16_t* dst, uint4 v) {
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(dst));
+}
+constexpr int kLinRows = 4;      // rows (waves) per workgroup
+constexpr int kPadGroups = 256;  // padding slots written at a time
 
-constexpr int kLinThreads = 512;
+// Calls put(s) for each of the slots rep_pos[p0], rep_pos[p0 + step], ... below p1; sid holds the first 64 of them,
+// one per lane. Every lane of the wave takes part.
+template <typename F>
+__device__ __forceinline__ void each_slot(const int* __restrict__ rep_pos, int p0, int p1, int step, int sid, F put) {
+  const int lane = threadIdx.x & 63;
+  for (int base = p0; base < p1; base += 64 * step) {
+    const int cnt = min(64, (p1 - base + step - 1) / step);
+    if (base != p0) sid = lane < cnt ? rep_pos[base + lane * step] : 0;
+    for (int j = 0; j < cnt; ++j) put((int64_t)__builtin_amdgcn_readlane(sid, j));
+  }
+}
 
 template <int RQ>
-__global__ void __launch_bounds__(kLinThreads) linattn_prep_k(const uint16_t* __restrict__ proj, const int4* __restrict__ hist,
-                                                     const int* __restrict__ rep_ptr, const int* __restrict__ rep_pos,
-                                                     const uint16_t* __restrict__ convw,
-                                                     const uint16_t* __restrict__ A_log,
-                                                     const uint16_t* __restrict__ dt_bias, uint16_t* __restrict__ q,
-                                                     uint16_t* __restrict__ k, uint16_t* __restrict__ v,
-                                                     float* __restrict__ g, uint16_t* __restrict__ beta, int N, int KD,
-                                                     int VD, int HV) {
+__global__ void __launch_bounds__(64 * kLinRows) linattn_prep_k(
+    const uint16_t* __restrict__ proj, const int4* __restrict__ hist, const int* __restrict__ rep_ptr,
+    const int* __restrict__ rep_pos, const uint16_t* __restrict__ convw, const uint16_t* __restrict__ A_log,
+    const uint16_t* __restrict__ dt_bias, uint16_t* __restrict__ q, uint16_t* __restrict__ k,
+    uint16_t* __restrict__ v, float* __restrict__ g, uint16_t* __restrict__ beta, int N, int KD, int VD, int HV) {
   constexpr int HD = 128;
-  extern __shared__ uint4 lds_raw[];
   const int C = 2 * KD + VD;
   const int64_t P = (int64_t)C + VD + 2 * HV;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = blockIdx.x;
-  const bool pad = n >= N;
-  const int4 hr = hist[min(n, N)];  // row N holds no history; issued beside the rep_ptr loads
-  int p0, p1;
-  if (!pad) {
-    p0 = rep_ptr[n];
-    p1 = rep_ptr[n + 1];
-  } else {
-    p0 = rep_ptr[N] + (n - N) * kPadSlots;
-    p1 = min(rep_ptr[N + 1], p0 + kPadSlots);
+  const int lane = threadIdx.x & 63;
+  const int rb = (N + kLinRows - 1) / kLinRows;  // row groups; padding groups follow
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int T = (C / 8 + 63) / 64 + 1;           // channel blocks of a row, the gates last
+  const int rg = blockIdx.x / T, cb = blockIdx.x - rg * T;
+  const bool pad = rg >= rb;
+  const int n = pad ? N : rg * kLinRows + wave;
+  if (n >= N && !pad) return;
+  int p0 = rep_ptr[n], step = 1;
+  const int p1 = rep_ptr[n + 1];
+  if (pad) {
+    p0 += (rg - rb) * kLinRows + wave;
+    step = kPadGroups;
   }
-  if (p0 >= p1) return;  // uniform over the workgroup
+  if (p0 >= p1) return;  // whole wave
+  const int sid = p0 + lane * step < p1 ? rep_pos[p0 + lane * step] : 0;
+  const int4 hr = hist[n];  // row N holds no history
 
-  uint16_t* orow = reinterpret_cast<uint16_t*>(lds_raw);                 // [C] bf16 bits
-  float* gl = reinterpret_cast<float*>(orow + C);                         // [HV] g
-  uint16_t* bl = reinterpret_cast<uint16_t*>(gl + HV);                    // [HV] beta bits
-  int* slot = reinterpret_cast<int*>(lds_raw) + (C * 2 + HV * 6 + 15) / 16 * 4;  // [kLinThreads] slot ids
-  // the first batch of slot ids is fetched now, so that its latency overlaps the row's compute
-  const int cnt0 = min(kLinThreads, p1 - p0);
-  const int sid0 = tid < cnt0 ? rep_pos[p0 + tid] : 0;
+  if (cb == T - 1) {  // the gates
+    for (int h0 = 0; h0 < HV; h0 += 64) {
+      const int h = h0 + lane;
+      const bool on = h < HV;
+      float gv = 0.f;
+      uint16_t bv = 0;
+      if (on && !pad) {
+        const uint16_t* br = proj + (int64_t)hr.w * P + C + VD;
+        bv = (uint16_t)f2bf(sigmoid_f(bf2f(br[h])));
+        const float xs = bf2f(br[HV + h]) + bf2f(dt_bias[h]);
+        gv = -expf(bf2f(A_log[h])) * (xs > 20.f ? xs : log1pf(expf(xs)));
+      }
+      each_slot(rep_pos, p0, p1, step, sid, [&](int64_t s) {
+        if (on) {
+          g[s * HV + h] = gv;
+          beta[s * HV + h] = bv;
+        }
+      });
+    }
+    return;
+  }
 
-  if (!pad) {
+  const int c0 = (cb * 64 + lane) * 8;
+  const bool live = c0 < C;
+  const bool isqk = c0 < 2 * KD;  // the same for all 16 lanes of a head (KD is a multiple of HD)
+  uint4 val = make_uint4(0u, 0u, 0u, 0u);
+  if (live && !pad) {
     const int rows[4] = {hr.x, hr.y, hr.z, hr.w};
-    for (int c0 = tid * 8; c0 < C; c0 += kLinThreads * 8) {
-      uint4 xr[4];
+    uint4 xr[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        xr[i] = rows[i] >= 0 ? *reinterpret_cast<const uint4*>(proj + (int64_t)rows[i] * P + c0)
-                             : make_uint4(0u, 0u, 0u, 0u);
-      const uint4* wp = reinterpret_cast<const uint4*>(convw + (int64_t)c0 * 4);  // [8 channels][4 taps]
-      const uint4 wq[4] = {wp[0], wp[1], wp[2], wp[3]};
-      const uint32_t* wv = &wq[0].x;
-      uint32_t packed[4];
+    for (int i = 0; i < 4; ++i)
+      xr[i] = rows[i] >= 0 ? *reinterpret_cast<const uint4*>(proj + (int64_t)rows[i] * P + c0)
+                           : make_uint4(0u, 0u, 0u, 0u);
+    const uint4* wp = reinterpret_cast<const uint4*>(convw + (int64_t)c0 * 4);  // [8 channels][4 taps]
+    const uint4 wq[4] = {wp[0], wp[1], wp[2], wp[3]};
+    const uint32_t* wv = &wq[0].x;
+    float o[8];
+    float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; j += 2) {
-        float o2[2];
+    for (int ch = 0; ch < 8; ++ch) {
+      float acc = 0.f;
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const int ch = j + jj;
-          float acc = 0.f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t* xw = &xr[i].x;
-            const float xv = bf2f((xw[ch >> 1] >> ((ch & 1) * 16)) & 0xffffu);
-            const int wi = ch * 4 + i;
-            const float wf = bf2f((wv[wi >> 1] >> ((wi & 1) * 16)) & 0xffffu);
-            acc += wf * xv;
-          }
-          o2[jj] = silu_f(acc);
-        }
-        packed[j >> 1] = pack2(o2[0], o2[1]);
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t* xw = &xr[i].x;
+        const float xv = bf2f((xw[ch >> 1] >> ((ch & 1) * 16)) & 0xffffu);
+        const int wi = ch * 4 + i;
+        const float wf = bf2f((wv[wi >> 1] >> ((wi & 1) * 16)) & 0xffffu);
+        acc += wf * xv;
       }
-      *reinterpret_cast<uint4*>(orow + c0) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+      o[ch] = rbf(silu_f(acc));
+      ss += o[ch] * o[ch];
     }
-    if (tid < HV) {
-      const uint16_t* br = proj + (int64_t)hr.w * P + C + VD;
-      bl[tid] = (uint16_t)f2bf(sigmoid_f(bf2f(br[tid])));
-      const float xs = bf2f(br[HV + tid]) + bf2f(dt_bias[tid]);
-      gl[tid] = -expf(bf2f(A_log[tid])) * (xs > 20.f ? xs : log1pf(expf(xs)));
+    if (isqk) {
+#pragma unroll
+      for (int off = 1; off < HD / 8; off <<= 1) ss += __shfl_xor(ss, off);
+      const float rs = 1.0f / sqrtf(ss + 1e-6f);
+#pragma unroll
+      for (int ch = 0; ch < 8; ++ch) o[ch] *= rs;
     }
-    __syncthreads();
-    // q / k heads: one per wave at a time, channels 2 lane, 2 lane + 1
-    for (int h = wave; h < 2 * KD / HD; h += kLinThreads / 64) {
-      uint32_t* pr = reinterpret_cast<uint32_t*>(orow + h * HD) + lane;
-      const uint32_t u = *pr;
-      const float a = bf2f(u & 0xffffu), b = bf2f(u >> 16);
-      float ss = a * a;
-      ss += b * b;
-      const float rs = 1.0f / sqrtf(wave_total(ss) + 1e-6f);
-      *pr = pack2(a * rs, b * rs);
-    }
+    val = make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
   }
-  __syncthreads();
-
-  // scatter: chunk u of a slot row is q (u < QC), k (QC <= u < 2 QC) or v; q/k rows hold each head RQ times
-  const int QC = RQ * KD / 8, VC = VD / 8, U = 2 * QC + VC;
-  for (int base = p0; base < p1; base += kLinThreads) {
-    const int cnt = min(kLinThreads, p1 - base);
-    if (tid < cnt) slot[tid] = base == p0 ? sid0 : rep_pos[base + tid];
-    __syncthreads();
-    for (int j = 0; j < cnt; ++j) {
-      const int64_t s = slot[j];
-      for (int u = tid; u < U; u += kLinThreads) {
-        uint4 val = make_uint4(0u, 0u, 0u, 0u);
-        uint16_t* dst;
-        int src;
-        if (u < 2 * QC) {
-          const bool isk = u >= QC;
-          const int e = (u - (isk ? QC : 0)) * 8;  // element within the RQ KD row
-          const int hk = e / (RQ * HD);
-          src = (isk ? KD : 0) + hk * HD + (e - hk * RQ * HD) % HD;
-          dst = (isk ? k : q) + s * (int64_t)(RQ * KD) + e;
-        } else {
-          const int e = (u - 2 * QC) * 8;
-          src = 2 * KD + e;
-          dst = v + s * (int64_t)VD + e;
-        }
-        if (!pad) val = *reinterpret_cast<const uint4*>(orow + src);
-        *reinterpret_cast<uint4*>(dst) = val;
-      }
-      if (tid < HV) {
-        g[s * HV + tid] = pad ? 0.f : gl[tid];
-        beta[s * HV + tid] = pad ? (uint16_t)0 : bl[tid];
-      }
+  // the lane's place in a slot's row: q / k rows hold each head RQ times side by side
+  const int64_t ld = isqk ? (int64_t)RQ * KD : VD;
+  const int cq = c0 < KD ? c0 : c0 - KD;
+  uint16_t* const dst = isqk ? (c0 < KD ? q : k) + (cq / HD) * (RQ * HD) + cq % HD : v + (c0 - 2 * KD);
+  each_slot(rep_pos, p0, p1, step, sid, [&](int64_t s) {
+    if (!live) return;
+    uint16_t* const d = dst + s * ld;
+    store_nt(d, val);
+    if (RQ > 1 && isqk) {
+#pragma unroll
+      for (int r = 1; r < RQ; ++r) store_nt(d + r * HD, val);
     }
-    __syncthreads();  // slot[] is refilled by the next batch
-  }
+  });
 }
 
 hipError_t launch_linattn_prep(const uint16_t* proj, const int32_t* hist, const int32_t* rep_ptr,
@@ -270,14 +269,13 @@ hipError_t launch_linattn_prep(const uint16_t* proj, const int32_t* hist, const 
                                const uint16_t* A_log, const uint16_t* dt_bias, int KD, int VD, int HV, int RQ,
                                uint16_t* q, uint16_t* k, uint16_t* v, float* g, uint16_t* beta, hipStream_t st) {
   const int C = 2 * KD + VD;
-  const size_t lds = (size_t)((C * 2 + HV * 6 + 15) / 16) * 16 + kLinThreads * sizeof(int);
-  const dim3 grid((unsigned)(N + (R + kPadSlots - 1) / kPadSlots));
-  if (RQ == 3)
-    hipLaunchKernelGGL(linattn_prep_k<3>, grid, dim3(kLinThreads), lds, st, proj, reinterpret_cast<const int4*>(hist),
-                       rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta, (int)N, KD, VD, HV);
-  else
-    hipLaunchKernelGGL(linattn_prep_k<1>, grid, dim3(kLinThreads), lds, st, proj, reinterpret_cast<const int4*>(hist),
-                       rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta, (int)N, KD, VD, HV);
+  const dim3 grid((unsigned)(((N + kLinRows - 1) / kLinRows + kPadGroups / kLinRows) * ((C / 8 + 63) / 64 + 1)));
+#define OJX_LIN(RQV)                                                                                                 \
+  hipLaunchKernelGGL(linattn_prep_k<RQV>, grid, dim3(64 * kLinRows), 0, st, proj, reinterpret_cast<const int4*>(hist), \
+                     rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta, (int)N, KD, VD, HV)
+  if (RQ == 3) OJX_LIN(3);
+  else OJX_LIN(1);
+#undef OJX_LIN
   return hipGetLastError();
 }
 

@@ -191,6 +191,29 @@ def test_linattn_prep_vs_oracle(ext, dev, tree, rep_qk):
         assert bool((tnsr.cpu()[pad] == 0).all())
 
 
+# A wave fetches slot ids 64 at a time, 256 waves share the padding slots, four rows share a workgroup and a wave
+# covers 512 channels: rows with 64, 65 and 130 slots, 300 padding slots and more, row counts off the group, channel
+# counts off the wave. Only the order of a head's sum of squares differs from the oracle's (one rounding step).
+@pytest.mark.parametrize("Lr,paths,short,HK,HV,PB,rep_qk", [(3, 64, 0, 1, 3, 1, True), (2, 65, 3, 1, 1, 16, False),
+                                                            (5, 130, 4, 2, 6, 16, True), (1, 7, 40, 3, 5, 8, False)])
+def test_linattn_prep_many_slots(ext, dev, Lr, paths, short, HK, HV, PB, rep_qk):
+    _say(f"case linattn_prep slots Lr={Lr} paths={paths} HK={HK} HV={HV} rep_qk={rep_qk}")
+    tree = (Lr, [0], [0] * paths, [1 + short] + [1] * (paths - 1))   # one long path pads all the others
+    LO, lay, proj, convw, A_log, dt_bias, KD, VD = _lin_inputs(tree, HK, HV, seed=paths, NB=1, PB=PB)
+    d = lambda a: torch.as_tensor(a).to(dev).contiguous()  # noqa: E731
+    args = (lay["hist"], lay["rep_ptr"], lay["rep_pos"])
+    got = ext.linattn_prep_dedup2(proj.to(dev), *map(d, args), lay["L2"], convw.to(dev), A_log.to(dev),
+                                  dt_bias.to(dev), KD, VD, HV, HK, 128, rep_qk)
+    want = LO.linattn_prep(proj, *args, lay["L2"], convw, A_log, dt_bias, KD, VD, HV, HK, 128, rep_qk)
+    for o, r, nm, steps in zip(got, want, "q k v g beta".split(), (2, 2, 1, 0, 1)):
+        if nm == "g":
+            assert torch.allclose(o.cpu(), r, rtol=2e-6, atol=0)
+        else:
+            _ulp_close(o, r, nm, min_equal=0.98, steps=steps)
+    pad = torch.as_tensor(lay["src"].reshape(-1) < 0)
+    assert all(bool((t.cpu()[pad] == 0).all()) for t in got)
+
+
 def test_linattn_prep_rejects(ext, dev):
     LO, lay, proj, convw, A_log, dt_bias, KD, VD = _lin_inputs(_TREES["nopad"], 2, 6, seed=1)
     d = lambda a: torch.as_tensor(a).to(dev).contiguous()  # noqa: E731
