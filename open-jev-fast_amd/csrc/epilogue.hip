@@ -79,7 +79,9 @@ __global__ void __launch_bounds__(256) reduce_silu_k(const float* __restrict__ p
 // One workgroup per row, H/8 threads, 8 contiguous elements per thread.
 // MODE 0: h = x (no add); 1: h = bf16(x + delta); 2: h = bf16(x + bf16(sum of the S fp32 planes)). HN: write hn.
 // Both are template parameters so that each variant is straight-line code and its loads (planes, x, w1) go out
-// together; the split-K variant runs on one workgroup per row, where memory latency is most of its time.
+// together; the split-K variant runs on one workgroup per row, where memory latency is most of its time. Bound at small
+// M by the launch and one memory latency (M = 7, 8 planes: 4.00 -> 3.91 us with the loads ahead of the planes and the
+// row sum without LDS shuffles), by its bytes at large M (norm alone, M = 539 4.4 -> 4.0, M = 2048 9.55 -> 8.75 us).
 template <int MODE, bool HN>
 __global__ void __launch_bounds__(1024) add_rmsnorm_k(const uint16_t* __restrict__ x,
                                                       const uint16_t* __restrict__ delta,
@@ -88,9 +90,19 @@ __global__ void __launch_bounds__(1024) add_rmsnorm_k(const uint16_t* __restrict
                                                       const int32_t* __restrict__ rowmask, float eps,
                                                       uint16_t* __restrict__ h_out, uint16_t* __restrict__ hn_out,
                                                       int H) {
-  __shared__ float red[16];
+  __shared__ float4 red[4];
   const int64_t row = blockIdx.x;
   const int i = threadIdx.x * 8;
+  // Everything that does not depend on the planes is requested before them: the plane loop has a run-time count, and
+  // loads placed after it would wait for it and cost a second memory latency.
+  const uint4 xa = *reinterpret_cast<const uint4*>(x + row * H + i);
+  float4 wa = make_float4(0.f, 0.f, 0.f, 0.f), wb = wa;
+  bool keep = true;
+  if constexpr (HN) {
+    wa = *reinterpret_cast<const float4*>(w1 + i);
+    wb = *reinterpret_cast<const float4*>(w1 + i + 4);
+    keep = rowmask == nullptr || rowmask[row] != 0;
+  }
   float d[8];
   if constexpr (MODE == 2) {
     float4 ab[2];
@@ -103,12 +115,6 @@ __global__ void __launch_bounds__(1024) add_rmsnorm_k(const uint16_t* __restrict
 #pragma unroll
     for (int j = 0; j < 4; ++j) { d[2 * j] = bf2f(dw[j] & 0xffffu); d[2 * j + 1] = bf2f(dw[j] >> 16); }
   }
-  const uint4 xa = *reinterpret_cast<const uint4*>(x + row * H + i);
-  float4 wa = make_float4(0.f, 0.f, 0.f, 0.f), wb = wa;
-  if constexpr (HN) {
-    wa = *reinterpret_cast<const float4*>(w1 + i);
-    wb = *reinterpret_cast<const float4*>(w1 + i + 4);
-  }
   const uint32_t xw[4] = {xa.x, xa.y, xa.z, xa.w};
   float v[8];
 #pragma unroll
@@ -119,7 +125,7 @@ __global__ void __launch_bounds__(1024) add_rmsnorm_k(const uint16_t* __restrict
     *reinterpret_cast<uint4*>(h_out + row * H + i) =
         make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
   }
-  if constexpr (HN) rmsnorm_row8(v, wa, wb, rowmask == nullptr || rowmask[row] != 0, eps, H, red, hn_out + row * H + i);
+  if constexpr (HN) rmsnorm_row8(v, wa, wb, keep, eps, H, red, hn_out + row * H + i);
 }
 
 __global__ void __launch_bounds__(256) silu_mul_k(const uint16_t* __restrict__ gu, const uint16_t* __restrict__ tab,

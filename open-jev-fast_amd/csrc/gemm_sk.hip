@@ -468,20 +468,34 @@ __global__ void __launch_bounds__(256) gemm_sk_fixup_kernel(const GemmParams p, 
   }
 }
 
+// The pieces of stream-K tile ts: workgroups g0 .. g1, first slot of g0 (all others start inside the tile: 2 g). In
+// 32-bit arithmetic where the products fit, which they do for every grid of the plans (a 64-bit division costs a few
+// hundred cycles, on the critical path of the row pass).
+template <typename I>
+__device__ __forceinline__ void sk_pieces(int ts, int ipt, int64_t T64, int64_t Gs64, int& g0, int& g1, int& slot0) {
+  const I T = (I)T64, Gs = (I)Gs64, x0 = (I)ts * (I)ipt;
+  const I a = ((x0 + 1) * Gs + T - 1) / T - 1;        // sk_owner(x0)
+  const I b = ((x0 + (I)ipt) * Gs + T - 1) / T - 1;   // sk_owner(x0 + ipt - 1)
+  g0 = (int)a;
+  g1 = (int)b;
+  slot0 = (int)(2 * a + (a * T / Gs >= x0 ? 0 : 1));  // sk_start(g0)
+}
+
 // Second pass of a stream-K plan with the residual epilogue, fused with the RMSNorm of the rows: one workgroup per
 // output row m, N/8 threads, 8 consecutive columns each. For a column of a split tile the thread sums the tile's
 // pieces in K order exactly as gemm_sk_fixup_kernel does and writes h = bf16(residual + bf16(sum)); columns of
 // tiles done whole were written by the GEMM and are read back. Then hn = RMSNorm(h) * w1 with the arithmetic of
 // add_rmsnorm_k, so the result is bit-identical to GEMM -> fixup -> add_rmsnorm in one launch fewer, with h not
 // read back for the split tiles (the reference: bmm, then add_rmsnorm_sk2, src/fastmodel.py:196-203).
+// One latency per pair of pieces, the residual, weights and mask requested ahead of them: o_proj M = 539 (spread 4)
+// 55.1 -> 53.2 us for GEMM and row pass, M = 1024 82.4 -> 80.1, down M = 1024 179.9 -> 177.9.
 template <int FN, int FM, int WN, int WM>
 __global__ void __launch_bounds__(1024) gemm_sk_fixup_rmsnorm_kernel(const GemmParams p, const float* w1,
                                                                     const int32_t* rowmask, float eps,
                                                                     uint16_t* hn_out) {
   constexpr int BN = WN * FN * 16, BM = WM * FM * 16, BK = 64;
-  __shared__ float red[16];
+  __shared__ float4 red[4];
   const int m = blockIdx.x, n8 = threadIdx.x * 8;
-  const int N = p.N;
   const int ipt = (p.K + BK - 1) / BK;
   const int64_t T = (int64_t)(p.tiles_n * p.tiles_m - p.dp_tiles) * ipt;
   const int64_t Gs = p.sk_grid;
@@ -489,45 +503,44 @@ __global__ void __launch_bounds__(1024) gemm_sk_fixup_rmsnorm_kernel(const GemmP
   const int tm = m / BM, mm = m % BM;
   const int tau = tn * p.tiles_m + tm;
   uint16_t* const h = static_cast<uint16_t*>(p.out) + (int64_t)m * p.ldo + n8;
-  float v[8];
   bool split = false;
-  int64_t g0 = 0, g1 = 0, x0 = 0;
+  int g0 = 0, g1 = 0, slot0 = 0;
   if (tau >= p.dp_tiles && T > 0) {
-    x0 = (int64_t)(tau - p.dp_tiles) * ipt;
-    g0 = sk_owner(x0, T, Gs);
-    g1 = sk_owner(x0 + ipt - 1, T, Gs);
+    if ((T + 1) * (Gs + 1) < (1LL << 31)) sk_pieces<uint32_t>(tau - p.dp_tiles, ipt, T, Gs, g0, g1, slot0);
+    else sk_pieces<int64_t>(tau - p.dp_tiles, ipt, T, Gs, g0, g1, slot0);
     split = g0 != g1;
   }
+  // a split tile's residual, or the h of a tile done whole: one load, in flight with the weights and the pieces
+  const uint4 xa = *reinterpret_cast<const uint4*>(split ? p.res + (int64_t)m * p.ldr + n8 : h);
+  const float4 wa = *reinterpret_cast<const float4*>(w1 + n8), wb = *reinterpret_cast<const float4*>(w1 + n8 + 4);
+  const bool keep = rowmask == nullptr || rowmask[m] != 0;
+  const uint32_t xw[4] = {xa.x, xa.y, xa.z, xa.w};
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { v[2 * e] = bf2f(xw[e] & 0xffffu); v[2 * e + 1] = bf2f(xw[e] >> 16); }
   if (split) {
     const float* base = p.sk_ws + (int64_t)mm * BN + c;  // row-major slots: columns c .. c+7 of tile row mm
-    auto slot = [&](int64_t g) { return (int64_t)(2 * g + (sk_start(g, T, Gs) >= x0 ? 0 : 1)) * (BN * BM); };
-    f32x4 a = *reinterpret_cast<const f32x4*>(base + slot(g0));
-    f32x4 b = *reinterpret_cast<const f32x4*>(base + slot(g0) + 4);
-    for (int64_t g = g0 + 1; g <= g1; ++g) {
-      const f32x4 ca = *reinterpret_cast<const f32x4*>(base + slot(g));
-      const f32x4 cb = *reinterpret_cast<const f32x4*>(base + slot(g) + 4);
+    auto at = [&](int64_t slot) { return reinterpret_cast<const f32x4*>(base + slot * (BN * BM)); };
+    f32x4 a = at(slot0)[0], b = at(slot0)[1];
+    int g = g0 + 1;
+    for (; g + 1 <= g1; g += 2) {  // two pieces in flight, added in K order
+      const f32x4 ca = at(2LL * g)[0], cb = at(2LL * g)[1], da = at(2LL * g + 2)[0], db = at(2LL * g + 2)[1];
       a += ca;
       b += cb;
+      a += da;
+      b += db;
     }
-    const uint4 ra = *reinterpret_cast<const uint4*>(p.res + (int64_t)m * p.ldr + n8);
-    const uint32_t rw[4] = {ra.x, ra.y, ra.z, ra.w};
+    if (g <= g1) {
+      a += at(2LL * g)[0];
+      b += at(2LL * g)[1];
+    }
     const float s[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[2 * e] = rbf(bf2f(rw[e] & 0xffffu) + rbf(s[2 * e]));
-      v[2 * e + 1] = rbf(bf2f(rw[e] >> 16) + rbf(s[2 * e + 1]));
-    }
+    for (int e = 0; e < 8; ++e) v[e] = rbf(v[e] + rbf(s[e]));
     *reinterpret_cast<uint4*>(h) = make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                               pack2(v[6], v[7]));
-  } else {
-    const uint4 ha = *reinterpret_cast<const uint4*>(h);
-    const uint32_t hw[4] = {ha.x, ha.y, ha.z, ha.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { v[2 * e] = bf2f(hw[e] & 0xffffu); v[2 * e + 1] = bf2f(hw[e] >> 16); }
   }
-  (void)N;
-  const float4 wa = *reinterpret_cast<const float4*>(w1 + n8), wb = *reinterpret_cast<const float4*>(w1 + n8 + 4);
-  rmsnorm_row8(v, wa, wb, rowmask == nullptr || rowmask[m] != 0, eps, p.N, red, hn_out + (int64_t)m * p.N + n8);
+  rmsnorm_row8(v, wa, wb, keep, eps, p.N, red, hn_out + (int64_t)m * p.N + n8);
 }
 
 }  // namespace ojx

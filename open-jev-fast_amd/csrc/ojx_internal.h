@@ -24,15 +24,52 @@ __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf
 
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return f2bf(a) | (f2bf(b) << 16); }
 
-// Sum over the whole workgroup (wave64 butterfly, then one value per wave through LDS).
-__device__ __forceinline__ float block_sum(float v, float* red) {
+// Sum over the wave's 64 lanes, in every lane: the xor butterfly 32, 16, 8, 4, 2, 1 without its six LDS round trips
+// (a __shfl_xor each). The lane swaps give each lane its partner's half; from step 8 down the values repeat every
+// 16, 8, 4, 2 lanes of a row, so that a rotation within the row of 16 brings the xor partner's value. Every addition
+// has the butterfly's two operands, hence its bits.
+__device__ __forceinline__ float wave_sum64(float v) {
+  typedef unsigned int u32p __attribute__((ext_vector_type(2)));
+  const unsigned int a = __float_as_uint(v);
+  const u32p h = __builtin_bit_cast(u32p, __builtin_amdgcn_permlane32_swap(a, a, false, false));
+  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const unsigned int b = __float_as_uint(v);
+  const u32p q = __builtin_bit_cast(u32p, __builtin_amdgcn_permlane16_swap(b, b, false, false));
+  v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+#define OJX_ROR(n) v += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x120 + (n), 0xf, 0xf, true))
+  OJX_ROR(8);
+  OJX_ROR(4);
+  OJX_ROR(2);
+  OJX_ROR(1);
+#undef OJX_ROR
+  return v;
+}
+
+// Sum over a workgroup of `threads` (at most 1024) threads: the wave sums, then one value per wave through LDS, added
+// in wave order. red holds 16 floats; the entries of absent waves are zero, so that four vector reads and a fixed
+// chain of additions serve every size. With a partial last wave the shuffles stay (they read absent lanes as zero).
+__device__ __forceinline__ float block_sum(float v, float4* red, int threads) {
+  const int nw = (threads + 63) >> 6;
+  if ((threads & 63) == 0) {
+    v = wave_sum64(v);
+  } else {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if (lane == 0) red[wid] = v;
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  }
+  float* const r = reinterpret_cast<float*>(red);
+  if (threadIdx.x == 0)
+    for (int i = nw; i < 16; ++i) r[i] = 0.f;
+  if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = v;
   __syncthreads();
   float t = 0.f;
-  for (int i = 0; i < nw; ++i) t += red[i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 c = red[i];
+    t += c.x;
+    t += c.y;
+    t += c.z;
+    t += c.w;
+  }
   return t;
 }
 
@@ -41,11 +78,11 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // src/kernels.cu:41-73). Each thread sums its own 8 squares in order, then block_sum: every kernel that normalises
 // a row this way gets the same bits.
 __device__ __forceinline__ void rmsnorm_row8(const float (&v)[8], float4 wa, float4 wb, bool keep, float eps, int H,
-                                             float* red, uint16_t* hn_dst) {
+                                             float4* red, uint16_t* hn_dst) {
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
-  ss = block_sum(ss, red);
+  ss = block_sum(ss, red, H >> 3);
   const float r = rsqrtf(ss / (float)H + eps);
   const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
   float o[8];

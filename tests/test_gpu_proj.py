@@ -269,6 +269,27 @@ def test_add_rmsnorm_variants(pkg, ext, O, dev):
         ext.add_rmsnorm_sk2(x.to(dev), torch.zeros(5, M, H, device=dev), w1.to(dev), None, 1e-6)
 
 
+# The row sum's shapes: a lone partial wave, whole waves (lane swaps and rotations instead of shuffles), whole waves
+# plus a partial one, and all 16 waves. hn depends on the sum of squares through one rsqrt: another order of its fp32
+# additions moves r by a few 2^-24, so at most a value on a rounding boundary moves, by one bf16 step.
+@pytest.mark.parametrize("H", [8, 56, 128, 512, 520, 1024, 4104, 5120, 8192])
+def test_rmsnorm_row_widths(ext, O, dev, H):
+    _say(f"case rmsnorm row H={H}")
+    g = torch.Generator().manual_seed(H)
+    M = 5
+    x = torch.randn(M, H, generator=g).bfloat16()
+    parts = torch.randn(7, M, H, generator=g).float()
+    w1 = (1.0 + 0.1 * torch.randn(H, generator=g)).float()
+    mask = torch.tensor([1, 0, 1, 1, 1], dtype=torch.int32)
+    for o, r in ((ext.add_rmsnorm(x.to(dev), None, w1.to(dev), mask.to(dev), 1e-6),
+                  O.add_rmsnorm(x, None, w1, mask, 1e-6)),
+                 (ext.add_rmsnorm_sk(x.to(dev), parts.to(dev), w1.to(dev), mask.to(dev), 1e-6),
+                  O.add_rmsnorm(x, None, w1, mask, 1e-6, parts=parts))):
+        assert torch.equal(o[0].cpu(), r[0])   # planes are added in the oracle's order
+        a, b = o[1].cpu().float(), r[1].float()
+        assert bool(((a - b).abs() <= b.abs() * 2.0 ** -7).all()) and bool((a[1] == 0).all())
+
+
 def test_silu_tables(pkg, ext, O, dev):
     _say("case act_tables")
     silu_b, sig_f = ext.act_tables(torch.empty(1, device=dev))
