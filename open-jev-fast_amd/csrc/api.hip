@@ -32,8 +32,18 @@ int hip_check(hipError_t e, const char* what) {
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int64_t kchunk_for(int64_t K, int64_t S) { return cdiv(cdiv(K, S), 8) * 8; }
-// split-K chunk over a packed weight: whole 64-k stages
+// split-K chunk of whole 64-k stages: required over a packed weight
 inline int64_t kchunk_pk(int64_t K, int64_t S) { return cdiv(cdiv(K, S), 64) * 64; }
+// Split-K chunk of a projection (its planes are reduced here, so where K is cut is this library's choice): whole 64-k
+// stages also for row-major operands, as long as every split then owns some K. A chunk that is only a multiple of 8
+// (K = 17408 in 6: 2904) starts each split's 128-byte row pieces off the cache lines, so that every stage reads two
+// lines for one, and ends each split in a partial stage: down row-major S = 6, M = 64 on tile 94 59.8 -> 40.5 us, M =
+// 288 on tile 81 90.7 -> 68.0.
+// ojx_gemm_splitk_f32 hands its planes out and keeps the equal K / S chunks of the reference's split weights.
+inline int64_t kchunk_proj(int64_t K, int64_t S) {
+  const int64_t c = kchunk_pk(K, S);
+  return (S - 1) * c < K ? c : kchunk_for(K, S);
+}
 inline bool is_packed_kind(int32_t kind) { return (kind & OJX_KIND_PACKED) != 0; }
 
 struct PlanEntry {
@@ -226,7 +236,8 @@ int check_dims(int64_t M, int64_t N, int64_t K) {
 int gemm(const ojx_cfg& c, int epi, const void* x, int64_t ldx, const void* w, int64_t ldw, void* out, int64_t ldo,
          const void* res, int64_t ldr, int64_t M, int64_t N, int64_t K, hipStream_t st, void* ws = nullptr,
          int64_t ws_off = 0, const float* w1 = nullptr, const int32_t* rowmask = nullptr, float eps = 0.f,
-         uint16_t* hn_out = nullptr, bool packed = false, const ojx::FattnParams* fa = nullptr) {
+         uint16_t* hn_out = nullptr, bool packed = false, const ojx::FattnParams* fa = nullptr,
+         bool equal_chunks = false) {
   const ojx::TileInfo* t = ojx::tile_info(c.tile);
   ojx::GemmParams p;
   p.fa = fa != nullptr ? *fa : ojx::FattnParams{};
@@ -242,7 +253,8 @@ int gemm(const ojx_cfg& c, int epi, const void* x, int64_t ldx, const void* w, i
   p.M = (int)M;
   p.N = (int)N;
   p.K = (int)K;
-  p.kchunk = (int)(packed ? kchunk_pk(K, c.splitk) : kchunk_for(K, c.splitk));
+  p.kchunk = (int)(packed ? kchunk_pk(K, c.splitk) : equal_chunks ? kchunk_for(K, c.splitk)
+                                                                  : kchunk_proj(K, c.splitk));
   p.wpk = packed ? 1 : 0;
   p.tiles_n = (int)cdiv(N, t->bn);
   p.tiles_m = (int)cdiv(M, t->bm);
@@ -458,7 +470,8 @@ int ojx_gemm_splitk_f32(const void* x, const void* w, float* parts, int64_t M, i
   c.one_launch = 0;  // planes out, no reduction
   if (!cfg_fits(M, N, K, c))
     return fail(OJX_ERR_CONFIG, "split-K S=%d (tile %d) invalid for K=%lld", S, c.tile, (long long)K);
-  return gemm(c, ojx::EPI_F32, x, ldx, w, ldw, parts, N, nullptr, 0, M, N, K, static_cast<hipStream_t>(stream));
+  return gemm(c, ojx::EPI_F32, x, ldx, w, ldw, parts, N, nullptr, 0, M, N, K, static_cast<hipStream_t>(stream), nullptr,
+              0, nullptr, nullptr, 0.f, nullptr, false, nullptr, true);
 }
 
 }  // extern "C"

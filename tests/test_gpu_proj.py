@@ -204,6 +204,24 @@ def test_mm_residual_rmsnorm_vs_oracle(pkg, ext, O, dev, M, N, K, masked):
                 assert bool((hn.cpu()[mask == 0] == 0).all())
 
 
+# Row-major K splits: cut at whole 64-k stages (328 / 6, 1096 / 16, 2904 / 6: the last split short), or, where that
+# would leave a split without K (200 / 5: 4 x 64 > 200; 136 / 4), into equal multiples of 8.
+@pytest.mark.parametrize("K,S", [(200, 5), (136, 4), (328, 6), (1096, 16), (2904, 6)])
+@pytest.mark.parametrize("tile", [0, 87])
+def test_row_major_split_chunks(ext, O, dev, K, S, tile):
+    _say(f"case split chunks K={K} S={S} tile={tile}")
+    g = torch.Generator().manual_seed(K + S)
+    M, N = 13, 264
+    x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * 0.05).bfloat16()
+    for ol in (0, 1):
+        _assert_tol(O, ext.mm(x.to(dev), w.to(dev), cfg=(tile, S, 0, 1, 0, ol)), O.linear_bf16(x, w), f"one launch {ol}")
+    res, w1 = torch.randn(M, N, generator=g).bfloat16(), torch.ones(N)
+    h, hn = ext.mm_residual_rmsnorm(res.to(dev), x.to(dev), w.to(dev), w1.to(dev), None, 1e-6, cfg=(tile, S))
+    rh, rhn = O.residual_proj(res, x, w, w1, None, 1e-6, S=S)
+    _assert_tol(O, h, rh, "h")
+    _assert_tol(O, hn, rhn, "hn")
+
+
 def test_splitk_parts_match_reference_chunks(pkg, ext, O, dev):
     """mm_splitk_f32 planes equal the reference's equal-K/S chunks (K % (8 S) == 0) within fp32 noise."""
     M, N, K, S = 64, 256, 2048, 4
