@@ -74,12 +74,7 @@ __device__ __forceinline__ void sk_sched() {  // NGA = groups before the barrier
 
 namespace {
 // The kernel body, specialised per epilogue mode (EPI) so that the epilogue is straight code for one mode.
-// NT: the weight DMAs carry the non-temporal hint. It is for a weight tile that one workgroup reads (a single M tile):
-// lines that several workgroups read are served more slowly with it (64 KB stages from L2: 98.5 against 67.4 us a call
-// in a probe of the DMA stream alone), and the M tiles of a weight tile read it within the same microsecond.
-// Measured over the plans of the projection shapes, hint against none: one M tile 0.975-0.99 of the time, two to
-// eight M tiles 1.00 (256 x 256) to 1.05 (256 x 128, 256 x 160, 256 x 192) of it.
-template <int FN, int FM, int WN, int WM, int EPI, bool PK, bool NT>
+template <int FN, int FM, int WN, int WM, int EPI, bool PK>
 __device__ __forceinline__ void sk_body(const GemmParams& p) {
   constexpr int BN = WN * FN * 16, BM = WM * FM * 16;
   constexpr int BK = 64, ROWS = BN + BM;
@@ -224,8 +219,7 @@ __device__ __forceinline__ void sk_body(const GemmParams& p) {
         uint32_t o_ = PK ? dWp0 : dW0 + i * stepW;                                                         \
         if (PK && n0 + BN > N && n0 + blk_ * 8 >= N) o_ = kOOB;                                            \
         if (partw_ && kw_ + kcol >= ke) o_ = kOOB;                                                         \
-        if constexpr (NT) dma16s_nt(rW_, wd_ + blk_ * 1024, o_, PK ? skp_ + (uint32_t)(i * (NW / 2 * 2048)) : skw_); \
-        else dma16s(rW_, wd_ + blk_ * 1024, o_, PK ? skp_ + (uint32_t)(i * (NW / 2 * 2048)) : skw_);        \
+        dma16s_nt(rW_, wd_ + blk_ * 1024, o_, PK ? skp_ + (uint32_t)(i * (NW / 2 * 2048)) : skw_);          \
       } else if (!(wonly)) {                                                                               \
         uint32_t o_ = real_ ? dX0 + (i - GW) * stepX : dXl;                                                \
         if (partx_ && kx_ + (real_ ? kcol : kcoll) >= ke) o_ = kOOB;                                       \
@@ -413,22 +407,17 @@ __device__ __forceinline__ void sk_body(const GemmParams& p) {
 
 }  // namespace
 
-template <int FN, int FM, int WN, int WM, int EPI>
-__device__ __forceinline__ void sk_dir(const GemmParams& p) {
-  if (p.wpk) {  // W in the packed layout
-    if (p.tiles_m == 1) sk_body<FN, FM, WN, WM, EPI, true, true>(p);
-    else sk_body<FN, FM, WN, WM, EPI, true, false>(p);
-  } else {
-    if (p.tiles_m == 1) sk_body<FN, FM, WN, WM, EPI, false, true>(p);
-    else sk_body<FN, FM, WN, WM, EPI, false, false>(p);
-  }
-}
-
 template <int FN, int FM, int WN, int WM>
 __global__ void __launch_bounds__(64 * WN * WM) gemm_sk_kernel(const GemmParams p, const int epi) {
-  if (epi == EPI_SILU) sk_dir<FN, FM, WN, WM, EPI_SILU>(p);
-  else if (epi == EPI_RESID) sk_dir<FN, FM, WN, WM, EPI_RESID>(p);
-  else sk_dir<FN, FM, WN, WM, EPI_BF16>(p);  // the host routes EPI_F32 (split-K planes) to other families
+  if (p.wpk) {  // W in the packed layout
+    if (epi == EPI_SILU) sk_body<FN, FM, WN, WM, EPI_SILU, true>(p);
+    else if (epi == EPI_RESID) sk_body<FN, FM, WN, WM, EPI_RESID, true>(p);
+    else sk_body<FN, FM, WN, WM, EPI_BF16, true>(p);  // the host routes EPI_F32 (split-K planes) to other families
+  } else {
+    if (epi == EPI_SILU) sk_body<FN, FM, WN, WM, EPI_SILU, false>(p);
+    else if (epi == EPI_RESID) sk_body<FN, FM, WN, WM, EPI_RESID, false>(p);
+    else sk_body<FN, FM, WN, WM, EPI_BF16, false>(p);
+  }
 }
 
 // Second pass of a stream-K plan: a tile that was split sums its pieces in K order, ((p0 + p1) + p2) + ..., and
