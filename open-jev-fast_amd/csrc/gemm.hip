@@ -215,22 +215,25 @@ __global__ void __launch_bounds__(64 * WN * WM) gemm_nt_kernel(const GemmParams 
 }
 
 // ------------------------------------------------------------------------------------------------ registry
-typedef void (*GemmFn)(const GemmParams, const int);
-
 struct TileEntry {
   TileInfo info;
-  GemmFn fn;
+  GemmFn (*pick)(int epi, bool packed);  // null: a retired id
   GemmFn fixup = nullptr;  // persistent family: second pass over the split stream-K tiles
   // persistent family: second pass fused with the residual RMSNorm (one workgroup per output row)
   void (*fixup_norm)(const GemmParams, const float*, const int32_t*, float, uint16_t*) = nullptr;
 };
 
+template <int BN, int BM, int BK, int WN, int WM>
+static GemmFn nt_pick(int epi, bool) {  // one kernel, epilogue and layout at run time
+  return epi >= EPI_BF16 && epi <= EPI_SILU ? gemm_nt_kernel<BN, BM, BK, WN, WM> : nullptr;
+}
+
 #define OJX_TILE(BN, BM, BK, WN, WM)                                                                         \
-  {{BN, BM, BK, WN, WM, 64 * WN * WM, 2 * (BN + BM) * (BK + 8) * 2, 0}, gemm_nt_kernel<BN, BM, BK, WN, WM>}
+  {{BN, BM, BK, WN, WM, 64 * WN * WM, 2 * (BN + BM) * (BK + 8) * 2, 0}, nt_pick<BN, BM, BK, WN, WM>}
 // Persistent stream-K tiles: BN = WN*FN*16 W rows, BM = WM*FM*16 x rows, 64-k stages, two or three LDS buffers
 #define OJX_SK(FN, FM, WN, WM)                                                                               \
   {{WN * FN * 16, WM * FM * 16, 64, WN, WM, 64 * WN * WM, sk_lds(WN * FN * 16, WM * FM * 16), 5},          \
-   gemm_sk_kernel<FN, FM, WN, WM>, gemm_sk_fixup_kernel<FN, FM, WN, WM>,                                   \
+   sk_pick<FN, FM, WN, WM>, gemm_sk_fixup_kernel<FN, FM, WN, WM>,                                          \
    gemm_sk_fixup_rmsnorm_kernel<FN, FM, WN, WM>}
 // Retired ids (16-72: register-streamed W, LDS-DMA and 32x32-MFMA tiles, slower than families 0, 5 and 6 on every
 // measured shape): kept so that stored ids keep their meaning; nothing plans, fits or launches them.
@@ -239,7 +242,7 @@ struct TileEntry {
 // stages (the prefetch distance) and a W ring of XD + 1
 #define OJX_KXD(FW, FX, XE, XD)                                                                              \
   {{16 * FW, 16 * (4 * FX + XE), 64, 4, 2, 512, ((XD + 1) * 16 * FW + XD * 16 * (4 * FX + XE)) * 128, 6},   \
-   gemm_kx_kernel<FW, FX, XE, XD>}
+   kx_pick<FW, FX, XE, XD>}
 #define OJX_KX(FW, FX, XE) OJX_KXD(FW, FX, XE, 2)
 
 // Order is the tile id used by the plan table; append only (ids are stored in plan_table.inc).
@@ -341,10 +344,10 @@ static const TileEntry kTiles[] = {
     OJX_KXD(8, 1, 0, 4),            // 94 128 x 64, DMAs 4 stages ahead (weight streaming at M = 64-128)
 };
 
-// Per device (the attribute is set with the device current) and per tile; threads that race here both set the same
-// attribute, which is harmless.
-constexpr int kAttrDevices = 64;
-static std::atomic<bool> g_attr_set[kAttrDevices][sizeof(kTiles) / sizeof(kTiles[0])];
+// Per device (the attribute is set with the device current), tile and kernel of the tile; threads that race here both
+// set the same attribute, which is harmless.
+constexpr int kAttrDevices = 64, kVariants = EPI_COUNT * 2;
+static std::atomic<bool> g_attr_set[kAttrDevices][sizeof(kTiles) / sizeof(kTiles[0])][kVariants];
 
 int num_tiles() { return (int)(sizeof(kTiles) / sizeof(kTiles[0])); }
 
@@ -353,35 +356,45 @@ const TileInfo* tile_info(int tile) {
   return &kTiles[tile].info;
 }
 
-static hipError_t set_attr(int tile) {
+static GemmFn kernel_of(int tile, int epi, bool packed) {
+  const TileEntry& e = kTiles[tile];
+  return e.pick != nullptr && epi >= 0 && epi < EPI_COUNT ? e.pick(epi, packed) : nullptr;
+}
+
+// The dynamic-LDS limit of one kernel of a tile, on the current device.
+static hipError_t set_attr(int tile, int epi, bool packed) {
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return err;
   if (dev < 0 || dev >= kAttrDevices) return hipErrorInvalidDevice;
-  std::atomic<bool>& done = g_attr_set[dev][tile];
+  std::atomic<bool>& done = g_attr_set[dev][tile][epi * 2 + (packed ? 1 : 0)];
   if (done.load(std::memory_order_acquire)) return hipSuccess;
-  const TileEntry& e = kTiles[tile];
-  if (e.fn != nullptr && e.info.lds_bytes != 0)  // not a retired id, and dynamic LDS
-    err = hipFuncSetAttribute(reinterpret_cast<const void*>(e.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              e.info.lds_bytes);
+  const GemmFn fn = kernel_of(tile, epi, packed);
+  if (fn != nullptr && kTiles[tile].info.lds_bytes != 0)
+    err = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kTiles[tile].info.lds_bytes);
   if (err == hipSuccess) done.store(true, std::memory_order_release);
   return err;
 }
 
 hipError_t init_tiles() {
-  for (int t = 0; t < num_tiles(); ++t) {
-    hipError_t err = set_attr(t);
-    if (err != hipSuccess) return err;
-  }
+  for (int t = 0; t < num_tiles(); ++t)
+    for (int v = 0; v < kVariants; ++v) {
+      hipError_t err = set_attr(t, v >> 1, (v & 1) != 0);
+      if (err != hipSuccess) return err;
+    }
   return hipSuccess;
 }
 
 static hipError_t launch_main(const TileEntry& e, int tile, int epi, const GemmParams& p, hipStream_t stream,
                               int grid) {
-  hipError_t err = set_attr(tile);
+  const bool packed = p.wpk != 0;
+  const GemmFn fn = kernel_of(tile, epi, packed);
+  if (fn == nullptr) return hipErrorInvalidValue;
+  hipError_t err = set_attr(tile, epi, packed);
   if (err != hipSuccess) return err;
   if (grid <= 0) grid = p.tiles_n * p.tiles_m * p.splits;
-  hipLaunchKernelGGL(e.fn, dim3(grid), dim3(e.info.threads), e.info.lds_bytes, stream, p, epi);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(e.info.threads), e.info.lds_bytes, stream, p, epi);
   return hipGetLastError();
 }
 
@@ -397,7 +410,7 @@ hipError_t launch_gemm_residual_rmsnorm_sk(int tile, const GemmParams& p, const 
 }
 
 hipError_t launch_gemm(int tile, int epi, const GemmParams& p, hipStream_t stream, int grid) {
-  if (tile < 0 || tile >= num_tiles() || kTiles[tile].fn == nullptr) return hipErrorInvalidValue;  // retired id
+  if (tile < 0 || tile >= num_tiles() || kTiles[tile].pick == nullptr) return hipErrorInvalidValue;  // retired id
   const TileEntry& e = kTiles[tile];
   hipError_t err = launch_main(e, tile, epi, p, stream, grid);
   if (err != hipSuccess || e.fixup == nullptr || p.sk_ws == nullptr) return err;

@@ -338,9 +338,14 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const int epi, c
 }  // namespace ojx
 
 namespace ojx {
+// The pick functions return a tile's kernel for an epilogue mode and weight layout, null where the tile has none; they
+// are instantiated beside the kernels. The persistent family has one kernel for each: a kernel that branches between
+// the bodies holds every body's scalars at once (256 x 256: 234 VGPRs and 47 spilled SGPRs with six bodies, 217-229
+// and none with one).
+typedef void (*GemmFn)(const GemmParams, const int epi);
 // Persistent stream-K family (gemm_sk.hip; instantiated there for the shapes of the tile table).
 template <int FN, int FM, int WN, int WM>
-__global__ void gemm_sk_kernel(const GemmParams p, const int epi);
+GemmFn sk_pick(int epi, bool packed);
 template <int FN, int FM, int WN, int WM>
 __global__ void gemm_sk_fixup_kernel(const GemmParams p, const int epi);
 template <int FN, int FM, int WN, int WM>
@@ -356,7 +361,7 @@ constexpr bool sk_asym(int BN, int BM) {
 constexpr int sk_lds(int BN, int BM) {
   return sk_asym(BN, BM) ? (3 * BN + 2 * BM) * 128 : sk_nbuf(BN, BM) * (BN + BM) * 128;
 }
-// K-interleaved wave pairs (gemm_kx.hip): BN x BM = 16 FW x 16 (4 FX + XE), 8 waves, x ring of XD stages.
+// K-interleaved wave pairs (gemm_kx.h): BN x BM = 16 FW x 16 (4 FX + XE), 8 waves, x ring of XD stages.
 template <int FW, int FX, int XE, int XD>
-__global__ void gemm_kx_kernel(const GemmParams p, const int epi);
+GemmFn kx_pick(int epi, bool packed);
 }  // namespace ojx

@@ -26,6 +26,7 @@
 //     MFMA group of the following groups.
 //   * A wave walks its W fragments starting at its first extra fragment (rotated order), so the extra MFMAs sit
 //     in the first EW groups of every stage for every wave: straight-line code for all groups.
+#pragma once
 #include "gemm_common.h"
 
 namespace ojx {
@@ -469,20 +470,12 @@ __global__ void __launch_bounds__(512) gemm_kx_kernel(const GemmParams p, const 
   else kx_dir<FW, FX, XE, XD, EPI_BF16>(p);
 }
 
-// Tile shapes of this family (registered in gemm.hip's tile table): BN x BM = 16 FW x 16 (4 FX + XE).
-template __global__ void gemm_kx_kernel<9, 4, 2, 2>(const GemmParams, const int);  // 144 x 288
-template __global__ void gemm_kx_kernel<8, 4, 2, 2>(const GemmParams, const int);  // 128 x 288
-template __global__ void gemm_kx_kernel<9, 2, 1, 2>(const GemmParams, const int);  // 144 x 144
-template __global__ void gemm_kx_kernel<8, 4, 0, 2>(const GemmParams, const int);  // 128 x 256
-template __global__ void gemm_kx_kernel<9, 1, 0, 2>(const GemmParams, const int);  // 144 x 64
-template __global__ void gemm_kx_kernel<9, 2, 0, 2>(const GemmParams, const int);  // 144 x 128
-template __global__ void gemm_kx_kernel<8, 2, 0, 2>(const GemmParams, const int);  // 128 x 128
-template __global__ void gemm_kx_kernel<8, 1, 0, 2>(const GemmParams, const int);  // 128 x 64
-template __global__ void gemm_kx_kernel<16, 2, 0, 2>(const GemmParams, const int);  // 256 x 128: one head per tile
-template __global__ void gemm_kx_kernel<16, 1, 0, 2>(const GemmParams, const int);  // 256 x 64
-template __global__ void gemm_kx_kernel<10, 4, 0, 2>(const GemmParams, const int);  // 160 x 256
-template __global__ void gemm_kx_kernel<10, 2, 0, 2>(const GemmParams, const int);  // 160 x 128
-// a deeper ring for the weight-streaming M = 64-128: twice the bytes in flight per CU
-template __global__ void gemm_kx_kernel<8, 1, 0, 4>(const GemmParams, const int);  // 128 x 64, 4 stages ahead
+// One kernel for every epilogue and layout: unlike the persistent family's, it gains nothing from being split (the
+// 144 x 288 and 128 x 288 tiles spill 120-360 registers in kernels of one epilogue, none here).
+template <int FW, int FX, int XE, int XD>
+GemmFn kx_pick(int epi, bool) {
+  const bool prep = FW == 16 && XE == 0;  // the 256-row tiles also carry the full-attention prep epilogue
+  return epi != EPI_FATTN || prep ? gemm_kx_kernel<FW, FX, XE, XD> : nullptr;
+}
 
 }  // namespace ojx

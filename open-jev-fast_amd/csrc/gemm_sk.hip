@@ -20,7 +20,7 @@
 //     stage: issued in one burst they fill the texture unit's command queue and stall the issuing waves.
 //   * The operand with fewer fragments per wave stays in registers for a stage; the other one's fragments are read
 //     two MFMA groups ahead, so LDS latency hides behind MFMAs.
-//   * The body is compiled once per epilogue mode. The epilogue stages the accumulators through LDS a few fragment
+//   * One kernel per epilogue mode and weight layout. The epilogue stages the accumulators through LDS a few fragment
 //     columns at a time and applies the mode in a short rolled loop (the fully unrolled form was instruction-fetch
 //     bound); its SiLU arithmetic is what remains of its cost.
 //   * Persistent grid of one workgroup per CU. Tiles are first handed out in whole-tile waves of G (one tile per
@@ -32,6 +32,8 @@
 //     another, and the GEMM carries no cross-workgroup code: an in-kernel last-arrival reduction was measured
 //     (its registers cost the main loop spills, and its coherent stores bypassing L2 cost more than a launch).
 #include "gemm_common.h"
+
+#include <type_traits>
 
 namespace ojx {
 
@@ -407,17 +409,25 @@ __device__ __forceinline__ void sk_body(const GemmParams& p) {
 
 }  // namespace
 
+// Two waves per SIMD are all that its LDS lets be resident; the compiler is told, so that it does not give up
+// instruction overlap for registers that no further wave could use. One kernel per mode and layout with this, against
+// one kernel that branches between six bodies, over the plans of gate-up, QKV and down at M = 64-2048: 256 x 128 1.3%,
+// 256 x 96 1%, 192 x 288 and 256 x 256 0.5% faster, the others level.
+template <int FN, int FM, int WN, int WM, int EPI, bool PK>
+__global__ void __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_sk_kernel(const GemmParams p, const int) {
+  sk_body<FN, FM, WN, WM, EPI, PK>(p);
+}
+
 template <int FN, int FM, int WN, int WM>
-__global__ void __launch_bounds__(64 * WN * WM) gemm_sk_kernel(const GemmParams p, const int epi) {
-  if (p.wpk) {  // W in the packed layout
-    if (epi == EPI_SILU) sk_body<FN, FM, WN, WM, EPI_SILU, true>(p);
-    else if (epi == EPI_RESID) sk_body<FN, FM, WN, WM, EPI_RESID, true>(p);
-    else sk_body<FN, FM, WN, WM, EPI_BF16, true>(p);  // the host routes EPI_F32 (split-K planes) to other families
-  } else {
-    if (epi == EPI_SILU) sk_body<FN, FM, WN, WM, EPI_SILU, false>(p);
-    else if (epi == EPI_RESID) sk_body<FN, FM, WN, WM, EPI_RESID, false>(p);
-    else sk_body<FN, FM, WN, WM, EPI_BF16, false>(p);
-  }
+GemmFn sk_pick(int epi, bool packed) {
+  auto of = [&](auto mode) -> GemmFn {
+    constexpr int E = decltype(mode)::value;
+    return packed ? gemm_sk_kernel<FN, FM, WN, WM, E, true> : gemm_sk_kernel<FN, FM, WN, WM, E, false>;
+  };
+  if (epi == EPI_BF16) return of(std::integral_constant<int, EPI_BF16>());
+  if (epi == EPI_RESID) return of(std::integral_constant<int, EPI_RESID>());
+  if (epi == EPI_SILU) return of(std::integral_constant<int, EPI_SILU>());
+  return nullptr;  // no K planes (EPI_F32): the host routes them to other families
 }
 
 // Second pass of a stream-K plan: a tile that was split sums its pieces in K order, ((p0 + p1) + p2) + ..., and
@@ -547,31 +557,31 @@ __global__ void __launch_bounds__(1024) gemm_sk_fixup_rmsnorm_kernel(const GemmP
 
 namespace ojx {
 // Tile shapes of this family (registered in gemm.hip's tile table): BN x BM = (WN*FN*16) x (WM*FM*16).
-template __global__ void gemm_sk_kernel<8, 4, 2, 4>(const GemmParams, const int);  // 256 x 256
+template GemmFn sk_pick<8, 4, 2, 4>(int, bool);  // 256 x 256
 template __global__ void gemm_sk_fixup_kernel<8, 4, 2, 4>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<8, 4, 2, 4>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<4, 9, 4, 2>(const GemmParams, const int);  // 256 x 288
+template GemmFn sk_pick<4, 9, 4, 2>(int, bool);  // 256 x 288
 template __global__ void gemm_sk_fixup_kernel<4, 9, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 9, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<4, 4, 4, 2>(const GemmParams, const int);  // 256 x 128
+template GemmFn sk_pick<4, 4, 4, 2>(int, bool);  // 256 x 128
 template __global__ void gemm_sk_fixup_kernel<4, 4, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 4, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<4, 6, 4, 2>(const GemmParams, const int);  // 256 x 192
+template GemmFn sk_pick<4, 6, 4, 2>(int, bool);  // 256 x 192
 template __global__ void gemm_sk_fixup_kernel<4, 6, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 6, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<4, 3, 4, 2>(const GemmParams, const int);  // 256 x 96
+template GemmFn sk_pick<4, 3, 4, 2>(int, bool);  // 256 x 96
 template __global__ void gemm_sk_fixup_kernel<4, 3, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 3, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<2, 9, 4, 2>(const GemmParams, const int);  // 128 x 288
+template GemmFn sk_pick<2, 9, 4, 2>(int, bool);  // 128 x 288
 template __global__ void gemm_sk_fixup_kernel<2, 9, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<2, 9, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
-template __global__ void gemm_sk_kernel<3, 9, 4, 2>(const GemmParams, const int);  // 192 x 288
+template GemmFn sk_pick<3, 9, 4, 2>(int, bool);  // 192 x 288
 template __global__ void gemm_sk_fixup_kernel<3, 9, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<3, 9, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
