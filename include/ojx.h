@@ -86,7 +86,8 @@ int ojx_init(void);
 int ojx_num_tiles(void);
 int ojx_tile_info(int32_t tile, int32_t* info7);
 
-/* Plan lookup for a shape: a static table measured offline on MI355X, with a heuristic for shapes not in it.
+/* Plan lookup for a shape: a static table measured offline on MI355X (single row counts and ranges of them), and for
+ * everything else the (tile, split) with the lowest estimated time.
  * Never times anything, so it is safe during graph capture.
  * Replaces the per-shape cuBLASLt heuristic/search: lt_setup (src/lt.cpp:15-42), _tune (src/fastmodel.py:114-132),
  * lt2_plan / lt2_search (src/lt.cpp:64-159). For OJX_KIND_SILU_MUL, N is the packed 2*I. */

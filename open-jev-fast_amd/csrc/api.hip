@@ -46,12 +46,13 @@ inline int64_t kchunk_proj(int64_t K, int64_t S) {
 }
 inline bool is_packed_kind(int32_t kind) { return (kind & OJX_KIND_PACKED) != 0; }
 
+// A row covers the calls of M rows (m_lo = 0) or of m_lo .. M rows.
 struct PlanEntry {
   int64_t M, N, K;
-  int32_t kind, tile, splitk, tail_tile, tail_splitk, tail_rows, one_launch;
+  int32_t kind, tile, splitk, tail_tile, tail_splitk, tail_rows, one_launch, m_lo;
 };
 
-// Measured on MI355X by the offline sweep (tuning script in the package); shapes not listed use heuristic_plan.
+// Measured on MI355X by the offline sweep (tuning script in the package); other calls use rule_plan.
 const PlanEntry kPlan[] = {
 #include "plan_table.inc"
 };
@@ -182,30 +183,90 @@ int64_t workspace_for(const ojx_cfg& c, int64_t M, int64_t N, int64_t K) {
   return parts[np - 1].ws + part_ws_bytes(parts[np - 1].c, M, parts[np - 1].n, K);
 }
 
-ojx_cfg heuristic_plan(int64_t M, int64_t N, int64_t K, int32_t kind) {
-  ojx_cfg c{};
-  if (is_packed_kind(kind)) {  // skinny tile, K-interleaved tile or persistent tile for the M range
-    c.tile = M <= 16 ? 0 : M <= 64 ? 84 : M <= 128 ? 85 : M <= 288 ? 80 : 73;
-    const ojx::TileInfo* t = ojx::tile_info(c.tile);
-    const int64_t tiles = cdiv(N, t->bn) * cdiv(M, t->bm);
-    int64_t S = 1;
-    while (S < 8 && tiles * S * 2 <= 320 && K / (S * 2) >= 512) S *= 2;
-    c.splitk = (int32_t)S;
-    while (c.splitk > 1 && !cfg_fits_packed(N, K, c)) --c.splitk;
-    return c;
+// The plan of every call that no table row covers: the (tile, split) with the lowest estimated time.
+//
+// Time of one 64-k stage of a tile with the whole chip running it (us). Fitted, with the constants of plan_us, to the
+// candidates within 30% of the best at 49 row counts (1-2048) of eight projection shapes and both weight layouts on
+// MI355X; picking by the estimate costs 2.4% of the best candidate's time on average there (8% at the 90th
+// percentile).
+struct StageCost {
+  int32_t tile;
+  double us;
+};
+constexpr StageCost kStageCost[] = {
+    {73, 1.462}, {74, 1.761}, {75, 0.861}, {76, 1.165}, {80, 1.178}, {81, 1.032}, {82, 0.843}, {83, 0.918},
+    {84, 0.498}, {85, 0.729}, {86, 0.650}, {92, 1.143}, {93, 0.714}, {94, 0.489}, {95, 0.531}, {96, 0.718},
+    {97, 0.883}, {98, 0.878}, {99, 0.996}, {100, 1.030}, {101, 1.346}, {102, 1.369}, {103, 0.688}, {104, 0.502}};
+constexpr int kRuleSplits[] = {1, 2, 3, 4, 6, 8};
+constexpr int64_t kPlanCus = 256;     // the plan does not depend on the machine that asks for it
+constexpr double kHbmBytesPerUs = 6.63e6;
+
+// Estimated time (us) of an M x N x K projection on tile t in S splits (persistent tiles: stream-K spread S; only
+// spreads that cut every remainder tile into S equal pieces are estimated, uneven ones measured up to 60% slower).
+// Rounds of one workgroup per CU, each its stages (at the tile's rate, or the weights' from HBM where that is slower)
+// plus a prologue and an epilogue; then the fp32 planes or pieces, written and read once, and the second launch (which
+// the residual projections run anyway, for their RMSNorm).
+double plan_us(const ojx::TileInfo* t, double stage, int64_t M, int64_t N, int64_t K, bool residual, int64_t S) {
+  const int64_t tm = cdiv(M, t->bm), tiles = cdiv(N, t->bn) * tm;
+  auto rate = [&](int64_t running) {  // us per stage with this many workgroups running
+    const double w = (double)std::min(running, kPlanCus) / (double)tm * t->bn * 128.0 / kHbmBytesPerUs;
+    return std::max(stage, w);
+  };
+  if (t->family == 5) {
+    const int64_t ipt = cdiv(K, 64), full = tiles / kPlanCus, rem = tiles - full * kPlanCus;
+    const int64_t gs = std::min(rem * S, rem * ipt);
+    const int64_t its = full * ipt + (rem > 0 ? cdiv(rem * ipt, gs) : 0);
+    double us = (double)its * rate(full > 0 ? kPlanCus : gs) + 9.82 * (double)(full + (rem > 0 ? 1 : 0));
+    if (gs > rem) us += (residual ? 0.0 : 5.21) + 2.0 * (double)(gs + rem) * t->bn * t->bm * 4.0 / 14.02e6;
+    return us;
   }
-  if (M <= 16) c.tile = 0;
-  else if (M <= 32) c.tile = 2;
-  else if (M <= 64) c.tile = 4;
-  else if (M <= 128) c.tile = 6;
-  else if (M <= 384) c.tile = 10;
-  else c.tile = 7;
-  const ojx::TileInfo* t = ojx::tile_info(c.tile);
-  const int64_t tiles = cdiv(N, t->bn) * cdiv(M, t->bm);
-  int64_t S = 1;
-  while (S < 8 && tiles * S * 2 <= 512 && K / (S * 2) >= 512) S *= 2;
-  c.splitk = (int32_t)S;
-  return c;
+  const int64_t nk = cdiv(cdiv(K, S), 64), wgs = tiles * S, rounds = cdiv(wgs, kPlanCus);
+  double us = (double)rounds * ((double)nk * rate(wgs) + 6.59);
+  if (S > 1) us += (residual ? 0.0 : 4.47) + 2.0 * (double)S * (double)M * (double)N * 4.0 / 8.44e6;
+  return us;
+}
+
+// The rule's plan. With planes > 0: the best tile that writes `planes` K planes, for callers that want the planes.
+// Splits only, no one-launch reduction: its arrival counters are shared between streams (see ol_counters), so it is
+// used where a table row names it and nowhere else.
+ojx_cfg rule_plan(int64_t M, int64_t N, int64_t K, int32_t kind, int32_t planes = 0) {
+  const bool packed = is_packed_kind(kind), residual = (kind & ~OJX_KIND_PACKED) == OJX_KIND_RESIDUAL;
+  M = std::max<int64_t>(M, 1);
+  ojx_cfg best{0, 1, 0, 1, 0, 0};
+  if (M <= 32 && !(M > 16 && cdiv(N, 144) >= 200)) {
+    // Weight streaming with 16- and 32-row tiles: as many K splits as bring the launch to about 500 workgroups (two
+    // per CU; three quarters of that or twice as many measured 3-10% slower on the 5120-row projections). From 200 W
+    // tiles of 144 rows on, M = 17-32 streams faster through the rule below (gate-up 55.5 against 64.6 us).
+    best.tile = M <= 16 ? 0 : 2;
+    const int64_t tiles = cdiv(N, ojx::tile_info(best.tile)->bn);
+    const int64_t s = std::min<int64_t>({8, 520 / tiles, K / 512});
+    best.splitk = planes > 0 ? planes : (int32_t)std::max<int64_t>(1, residual && N > 8192 ? 1 : s);
+    while (planes == 0 && best.splitk > 1 && !cfg_fits(M, N, K, best, packed)) --best.splitk;
+    return best;
+  }
+  double best_us = 0.0;
+  bool found = false;
+  for (const StageCost& sc : kStageCost) {
+    const ojx::TileInfo* t = ojx::tile_info(sc.tile);
+    const int64_t tiles = cdiv(N, t->bn) * cdiv(M, t->bm), rem = tiles % kPlanCus;
+    for (int32_t S : kRuleSplits) {
+      if (planes > 0) {
+        if (S > 1 || t->family == 5) break;
+        S = planes;
+      } else if (S > 1) {
+        if (t->family == 5 ? (rem == 0 || rem * S > kPlanCus) : (K / S < 512 || (residual && N > 8192))) break;
+      }
+      const ojx_cfg c{sc.tile, S, 0, 1, 0, 0};
+      const double us = plan_us(t, sc.us, M, N, K, residual, S);
+      if ((!found || us < best_us) && cfg_fits(M, N, K, c, packed)) {
+        best = c;
+        best_us = us;
+        found = true;
+      }
+    }
+  }
+  if (planes > 0) best.splitk = planes;
+  return best;
 }
 
 int resolve(int64_t M, int64_t N, int64_t K, int32_t kind, const ojx_cfg* cfg, ojx_cfg* out) {
@@ -399,13 +460,13 @@ int ojx_plan(int64_t M, int64_t N, int64_t K, int32_t kind, ojx_cfg* out) {
     return fail(OJX_ERR_ARG, "unknown kind %d", kind);
   const bool packed = is_packed_kind(kind);
   for (const PlanEntry& e : kPlan) {
-    if (e.M == M && e.N == N && e.K == K && e.kind == kind) {
+    if (e.N == N && e.K == K && e.kind == kind && (e.M == M || (e.m_lo > 0 && e.m_lo <= M && M <= e.M))) {
       ojx_cfg c{e.tile, e.splitk, e.tail_tile, e.tail_splitk, e.tail_rows, e.one_launch};
       if (c.tail_splitk == 0) c.tail_splitk = 1;
       if (cfg_fits(M, N, K, c, packed)) { *out = c; return OJX_OK; }
     }
   }
-  *out = heuristic_plan(M, N, K, kind);
+  *out = rule_plan(M, N, K, kind);
   if (!cfg_fits(M, N, K, *out, packed)) *out = ojx_cfg{out->tile, 1, 0, 1, 0};
   return OJX_OK;
 }
@@ -460,7 +521,7 @@ int ojx_gemm_splitk_f32(const void* x, const void* w, float* parts, int64_t M, i
   ojx_cfg c{};
   if (tile < 0) {
     OJX_TRY(ojx_plan(M, N, K, OJX_KIND_RESIDUAL, &c));
-    if (is_sk(c.tile)) c = heuristic_plan(M, N, K, OJX_KIND_RESIDUAL);  // that family writes no K planes
+    if (is_sk(c.tile)) c = rule_plan(M, N, K, OJX_KIND_RESIDUAL, S);  // that family writes no K planes
   } else {
     c.tile = tile;
   }

@@ -342,6 +342,16 @@ static const TileEntry kTiles[] = {
     OJX_KX(10, 4, 0),               // 92 160 x 256: N = 5120 in 32 W tiles, 256 tiles at M = 2048
     OJX_KX(10, 2, 0),               // 93 160 x 128: 256 tiles at M = 1024
     OJX_KXD(8, 1, 0, 4),            // 94 128 x 64, DMAs 4 stages ahead (weight streaming at M = 64-128)
+    OJX_KX(8, 1, 2),                // 95 128 x 96: N = 5120 at M = 65-112, two workgroups per CU
+    OJX_KX(8, 2, 2),                // 96 128 x 160
+    OJX_KX(9, 3, 0),                // 97 144 x 192: 242 W tiles of the gate-up at M <= 192
+    OJX_KX(8, 3, 2),                // 98 128 x 224
+    OJX_KX(9, 3, 2),                // 99 144 x 224
+    OJX_SK(4, 5, 4, 2),             // 100 256 x 160 persistent
+    OJX_SK(4, 7, 4, 2),             // 101 256 x 224
+    OJX_SK(6, 5, 2, 4),             // 102 192 x 320
+    OJX_SK(4, 3, 2, 4),             // 103 128 x 192
+    OJX_SK(2, 4, 4, 2),             // 104 128 x 128
 };
 
 // Per device (the attribute is set with the device current), tile and kernel of the tile; threads that race here both

@@ -7,4 +7,5 @@ template GemmFn kx_pick<9, 4, 2, 2>(int, bool);  // 144 x 288
 template GemmFn kx_pick<8, 4, 2, 2>(int, bool);  // 128 x 288
 template GemmFn kx_pick<8, 4, 0, 2>(int, bool);  // 128 x 256
 template GemmFn kx_pick<10, 4, 0, 2>(int, bool);  // 160 x 256
+template GemmFn kx_pick<9, 3, 0, 2>(int, bool);  // 144 x 192
 }  // namespace ojx

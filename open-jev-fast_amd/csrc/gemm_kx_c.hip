@@ -8,4 +8,5 @@ template GemmFn kx_pick<9, 2, 0, 2>(int, bool);  // 144 x 128
 template GemmFn kx_pick<8, 2, 0, 2>(int, bool);  // 128 x 128
 template GemmFn kx_pick<8, 1, 0, 2>(int, bool);  // 128 x 64
 template GemmFn kx_pick<8, 1, 0, 4>(int, bool);  // 128 x 64, 4 stages ahead
+template GemmFn kx_pick<8, 1, 2, 2>(int, bool);  // 128 x 96
 }  // namespace ojx

@@ -585,4 +585,24 @@ template GemmFn sk_pick<3, 9, 4, 2>(int, bool);  // 192 x 288
 template __global__ void gemm_sk_fixup_kernel<3, 9, 4, 2>(const GemmParams, const int);
 template __global__ void gemm_sk_fixup_rmsnorm_kernel<3, 9, 4, 2>(const GemmParams, const float*, const int32_t*,
                                                                   float, uint16_t*);
+template GemmFn sk_pick<4, 5, 4, 2>(int, bool);  // 256 x 160
+template __global__ void gemm_sk_fixup_kernel<4, 5, 4, 2>(const GemmParams, const int);
+template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 5, 4, 2>(const GemmParams, const float*, const int32_t*,
+                                                                  float, uint16_t*);
+template GemmFn sk_pick<4, 7, 4, 2>(int, bool);  // 256 x 224
+template __global__ void gemm_sk_fixup_kernel<4, 7, 4, 2>(const GemmParams, const int);
+template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 7, 4, 2>(const GemmParams, const float*, const int32_t*,
+                                                                  float, uint16_t*);
+template GemmFn sk_pick<6, 5, 2, 4>(int, bool);  // 192 x 320
+template __global__ void gemm_sk_fixup_kernel<6, 5, 2, 4>(const GemmParams, const int);
+template __global__ void gemm_sk_fixup_rmsnorm_kernel<6, 5, 2, 4>(const GemmParams, const float*, const int32_t*,
+                                                                  float, uint16_t*);
+template GemmFn sk_pick<4, 3, 2, 4>(int, bool);  // 128 x 192
+template __global__ void gemm_sk_fixup_kernel<4, 3, 2, 4>(const GemmParams, const int);
+template __global__ void gemm_sk_fixup_rmsnorm_kernel<4, 3, 2, 4>(const GemmParams, const float*, const int32_t*,
+                                                                  float, uint16_t*);
+template GemmFn sk_pick<2, 4, 4, 2>(int, bool);  // 128 x 128
+template __global__ void gemm_sk_fixup_kernel<2, 4, 4, 2>(const GemmParams, const int);
+template __global__ void gemm_sk_fixup_rmsnorm_kernel<2, 4, 4, 2>(const GemmParams, const float*, const int32_t*,
+                                                                  float, uint16_t*);
 }  // namespace ojx

@@ -62,6 +62,54 @@ def test_plan_table_names_live_tiles(pkg):
             assert pkg._lib.tile_info(t)["family"] >= 0, f"plan row {r} names tile {t}"
 
 
+def _plan_kinds(N, K):
+    return [k | p for k in (0, 1, 2) for p in (0, 4) if not p or (N % 16 == 0 and K % 64 == 0)]
+
+
+def test_plan_rule_off_the_table(pkg):
+    """Calls that no row covers: over sizes from one row and eight columns up, every plan is a configuration that the
+    library itself accepts (ojx_workspace_bytes checks it), names a live tile, has no tail and no one-launch
+    reduction, and leaves a residual projection wider than 8192 columns without planes (its row pass cannot read
+    them back without an RMSNorm output)."""
+    import random
+    rng = random.Random(3)
+    sizes = [(1, 8, 8), (17, 8, 8), (33, 16, 64), (2049, 5120, 5120), (65536, 256, 64), (300, 65536, 128)]
+    for _ in range(400):
+        M = int(2 ** rng.uniform(0, 13))
+        N = 16 * int(2 ** rng.uniform(0, 11)) if rng.random() < 0.5 else 8 * rng.randint(1, 4000)
+        K = 64 * rng.randint(1, 300) if rng.random() < 0.5 else 8 * rng.randint(1, 2500)
+        sizes.append((M, N, K))
+    for M, N, K in sizes:
+        for kind in _plan_kinds(N, K):
+            if kind & 4 and N * K * 2 >= 2 ** 31:
+                continue
+            c = pkg._lib.plan(M, N, K, kind)
+            what = (M, N, K, kind, c)
+            assert pkg._lib.tile_info(c.tile)["family"] in (0, 5, 6), what
+            assert pkg._lib.lib().ojx_workspace_bytes(M, N, K, kind, ctypes.byref(c)) >= 0, what
+            assert c.tail_rows == 0 and c.one_launch == 0 and 1 <= c.splitk <= 8, what
+            if kind & 3 == 2 and N > 8192 and pkg._lib.tile_info(c.tile)["family"] != 5:
+                assert c.splitk == 1, what
+
+
+def test_plan_table_ranges(pkg):
+    """Range rows (m_lo > 0): ordered, disjoint per shape and kind, two-launch, and the plan of every row count in
+    them; a row for a single count inside a range goes first."""
+    src = os.path.join(os.path.dirname(pkg.__file__), "csrc", "plan_table.inc")
+    rows = [list(map(int, m.group(1).split(","))) for m in re.finditer(r"^\{([^}]*)\}", open(src).read(), re.M)]
+    single = {tuple(r[:4]): (r[4], r[5], r[9]) for r in rows if len(r) < 11 or r[10] == 0}
+    last = {}
+    for r in rows:
+        if len(r) < 11 or r[10] == 0:
+            continue
+        hi, N, K, kind, lo = r[0], r[1], r[2], r[3], r[10]
+        assert 1 < lo <= hi and lo > last.get((N, K, kind), 0) and r[8] == 0 and r[9] == 0
+        last[(N, K, kind)] = hi
+        for M in (lo, (lo + hi) // 2, hi):
+            c = pkg._lib.plan(M, N, K, kind)
+            assert (c.tile, c.splitk, c.one_launch) == single.get((M, N, K, kind), (r[4], r[5], 0))
+
+
 @pytest.mark.parametrize("kind", [0, 1, 2, 4, 5, 6])
 def test_plan_valid_for_every_contract_shape(pkg, kind):
     L = pkg._lib.lib()

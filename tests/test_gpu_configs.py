@@ -79,6 +79,36 @@ def test_unpack_inverts_pack(O):
 
 
 # --------------------------------------------------------------------------------------- every plan-table row
+# Row counts between the table's single rows: range rows and the rule, at the edges of the tiles they choose
+# (M = 32 / 33, 96 / 97, 160, 192 / 193, 224, 320 / 321, 384, 640, 641), past the table (2049) and on a shape no row
+# names; the last rows of a partial M tile and the last columns of a partial N tile are in every comparison.
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M,N,K,kind", [
+    (17, 5120, 6144, 2), (32, 14336, 5120, 0), (33, 5120, 17408, 2), (96, 5120, 6144, 2), (97, 16480, 5120, 0),
+    (160, 5120, 17408, 2), (192, 34816, 5120, 1), (193, 34816, 5120, 1), (224, 16480, 5120, 0), (320, 34816, 5120, 1),
+    (321, 14336, 5120, 0), (384, 34816, 5120, 0), (640, 5120, 17408, 2), (641, 5120, 5120, 0), (832, 5120, 6144, 2),
+    (1153, 16480, 5120, 0), (2049, 5120, 6144, 2), (300, 2064, 3136, 0), (75, 4112, 1088, 1), (530, 1040, 4160, 2)])
+def test_plan_between_rows(pkg, ext, O, dev, M, N, K, kind, packed):
+    plan = pkg._lib.plan(M, N, K, kind | (4 if packed else 0))
+    _say(f"case off the rows M={M} N={N} K={K} kind={kind} packed={packed} plan={plan}")
+    gx = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=gx, device=dev).bfloat16()
+    w = weight(N, K, dev)
+    wk = ext.pack_weight(w) if packed else w
+    if kind == 0:
+        _assert_tol(O, ext.mm(x, wk), O.linear_bf16(x, w), "y")
+    elif kind == 1:
+        _assert_tol(O, ext.mm_silu_mul(x, wk), O.gate_up_silu(x, *unpack_gate_up(w)), "out")
+    else:
+        res = torch.randn(M, N, generator=gx, device=dev).bfloat16()
+        w1 = (1.0 + 0.1 * torch.randn(N, generator=gx, device=dev)).float()
+        mask = (torch.rand(M, generator=gx, device=dev) > 0.2).int()
+        h, hn = ext.mm_residual_rmsnorm(res, x, wk, w1, mask, 1e-6)
+        rh, rhn = ext.add_rmsnorm(res, O.linear_bf16(x, w), w1, mask, 1e-6)
+        _assert_tol(O, h, rh, "h")
+        _assert_tol(O, hn, rhn, "hn")
+
+
 @pytest.mark.parametrize("M,N,K,kind", plan_rows(), ids=lambda v: str(v))
 def test_plan_table_row_full_size(pkg, ext, O, dev, M, N, K, kind):
     """Rows of kind | 4 are plans for packed weights: the call goes through the *_pk entry point. Sampled rows and
