@@ -7,18 +7,19 @@ namespace ojx {
 
 namespace {
 
-// Sum over the 64 lanes of a wave (every lane gets the total).
-__device__ __forceinline__ float wave_total(float v) {
+__device__ __forceinline__ void unpack8(uint4 a, float (&v)[8]) {
+  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
-  return v;
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = bf2f(w[j] & 0xffffu);
+    v[2 * j + 1] = bf2f(w[j] >> 16);
+  }
 }
 
-__device__ __forceinline__ void unpack4(uint2 a, float (&v)[4]) {
-  v[0] = bf2f(a.x & 0xffffu);
-  v[1] = bf2f(a.x >> 16);
-  v[2] = bf2f(a.y & 0xffffu);
-  v[3] = bf2f(a.y >> 16);
+// Non-temporal store of a lane's 16 bytes: for output lines that are written whole and read by another kernel.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store_nt(uint16_t* dst, uint4 v) {
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(dst));
 }
 
 }  // namespace
@@ -34,11 +35,15 @@ __device__ __forceinline__ void unpack4(uint2 a, float (&v)[4]) {
 //   d < RD/2 and xn[d - RD/2] for RD/2 <= d < RD; dims >= RD keep xn.
 //   Outputs: qt [HQ, N, D], kt [HKV, N, D], vt [HKV, N, D] (head-major for attention) and gate [N, HQ D].
 //
-// Work layout: one wave per (token, head task), four tasks per workgroup. Task t of a token: t < HQ the q head t
-// (the wave also copies gate head t), HQ <= t < HQ + HKV the k head t - HQ, then the v heads (copies). Lane l owns
-// dims 4l .. 4l+3 (one 8-byte load, one 8-byte store: 512 contiguous bytes per wave). A q/k head's sum of squares
-// is a 64-lane wave total; the normalised head goes to the wave's own 1 KB of LDS, from which each lane of the
-// rotary part reads its four partner values xn[d -+ RD/2] (a wave-local exchange: no workgroup barrier).
+// Work layout: half a wave per (token, head task), eight tasks per workgroup. Task t of a token: t < HQ the q head t
+// (the half wave also copies gate head t), HQ <= t < HQ + HKV the k head t - HQ, then the v heads (copies). Lane l of
+// the 32 owns dims 8l .. 8l+7: one 16-byte load and store each, 512 contiguous bytes per head. A q/k head's sum of
+// squares is five shuffles; the rotary partner dims d -+ RD/2 are all held by lane l ^ (RD / 16) (RD is 16 times a power
+// of two), so the exchange is a shuffle of the eight values: no LDS, no barrier.
+// What bounds it: the launch up to a few hundred tokens, then its bytes. Stores are non-temporal (whole lines, read by
+// another kernel). Graph replays over rotating inputs; an earlier kernel (a wave of 8-byte lanes per task, the partner
+// through LDS, plain stores) -> the same with non-temporal stores -> this: M = 288 6.6 -> 6.1 -> 5.4 us, M = 539 9.4 ->
+// 8.6 -> 7.5, M = 1024 15.2 -> 13.5 -> 12.2 (4.8 TB/s), M = 2048 31.1 -> 30.4 -> 23.0 (5.1 TB/s); M = 7 2.7 -> 2.9.
 __global__ void __launch_bounds__(256) fullattn_prep_k(const uint16_t* __restrict__ proj, int64_t N, int HQ, int HKV,
                                                        int RD, float eps, const float* __restrict__ qw1,
                                                        const float* __restrict__ kw1, const uint16_t* __restrict__ cosb,
@@ -46,65 +51,63 @@ __global__ void __launch_bounds__(256) fullattn_prep_k(const uint16_t* __restric
                                                        uint16_t* __restrict__ kt, uint16_t* __restrict__ vt,
                                                        uint16_t* __restrict__ gate) {
   constexpr int D = 256;
-  __shared__ float4 xn_lds[4][D / 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int T = HQ + 2 * HKV, G = (T + 3) >> 2;  // tasks per token, workgroups per token
+  const int l = threadIdx.x & 31;
+  const int T = HQ + 2 * HKV, G = (T + 7) >> 3;  // tasks per token, workgroups per token
   const int64_t n = blockIdx.x / G;
-  const int t = (int)(blockIdx.x - n * G) * 4 + wave;
-  if (t >= T) return;  // whole wave; no workgroup barrier follows
+  const int t = (int)(blockIdx.x - n * G) * 8 + (threadIdx.x >> 5);
+  if (t >= T) return;  // whole half wave; the shuffles below stay within one
   const int64_t P = (int64_t)(2 * HQ + 2 * HKV) * D;
   const uint16_t* row = proj + n * P;
-  const int d0 = lane * 4;
+  const int d0 = l * 8;
   if (t >= HQ + HKV) {  // v head: a copy into [HKV, N, D]
     const int hv = t - HQ - HKV;
-    *reinterpret_cast<uint2*>(vt + ((int64_t)hv * N + n) * D + d0) =
-        *reinterpret_cast<const uint2*>(row + (int64_t)(2 * HQ + HKV) * D + hv * D + d0);
+    store_nt(vt + ((int64_t)hv * N + n) * D + d0,
+             *reinterpret_cast<const uint4*>(row + (int64_t)(2 * HQ + HKV) * D + hv * D + d0));
     return;
   }
   const bool isq = t < HQ;
+  const uint4 xa = *reinterpret_cast<const uint4*>(
+      row + (isq ? (int64_t)t * 2 * D : (int64_t)2 * HQ * D + (int64_t)(t - HQ) * D) + d0);
   if (isq)  // gate head: a copy into [N, HQ D]
-    *reinterpret_cast<uint2*>(gate + n * (int64_t)(HQ * D) + t * D + d0) =
-        *reinterpret_cast<const uint2*>(row + (int64_t)t * 2 * D + D + d0);
-  float x[4];
-  unpack4(*reinterpret_cast<const uint2*>(row + (isq ? (int64_t)t * 2 * D : (int64_t)2 * HQ * D + (int64_t)(t - HQ) * D)
-                                          + d0), x);
-  float ss = x[0] * x[0];
-  ss += x[1] * x[1];
-  ss += x[2] * x[2];
-  ss += x[3] * x[3];
-  const float r = rsqrtf(wave_total(ss) / (float)D + eps);
-  const float4 w = *reinterpret_cast<const float4*>((isq ? qw1 : kw1) + d0);
-  float xn[4];
-  xn[0] = rbf((x[0] * r) * w.x);
-  xn[1] = rbf((x[1] * r) * w.y);
-  xn[2] = rbf((x[2] * r) * w.z);
-  xn[3] = rbf((x[3] * r) * w.w);
-  float o[4] = {xn[0], xn[1], xn[2], xn[3]};
-  if (RD > 0) {
-    xn_lds[wave][lane] = make_float4(xn[0], xn[1], xn[2], xn[3]);
-    // the wave's LDS writes are complete and visible to its own lanes before the partner reads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (d0 < RD) {
-      float cs[4], sn[4];
-      unpack4(*reinterpret_cast<const uint2*>(cosb + n * RD + d0), cs);
-      unpack4(*reinterpret_cast<const uint2*>(sinb + n * RD + d0), sn);
-      const bool lo = d0 < RD / 2;
-      const float4 pq = xn_lds[wave][(lo ? d0 + RD / 2 : d0 - RD / 2) >> 2];
-      const float pv[4] = {pq.x, pq.y, pq.z, pq.w};
+    store_nt(gate + n * (int64_t)(HQ * D) + t * D + d0,
+             *reinterpret_cast<const uint4*>(row + (int64_t)t * 2 * D + D + d0));
+  const float* w1 = (isq ? qw1 : kw1) + d0;
+  const float4 wa = *reinterpret_cast<const float4*>(w1), wb = *reinterpret_cast<const float4*>(w1 + 4);
+  const bool rot = d0 < RD;
+  uint4 ca = make_uint4(0u, 0u, 0u, 0u), sa = ca;
+  if (rot) {
+    ca = *reinterpret_cast<const uint4*>(cosb + n * RD + d0);
+    sa = *reinterpret_cast<const uint4*>(sinb + n * RD + d0);
+  }
+  float x[8];
+  unpack8(xa, x);
+  float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = rbf(rbf(xn[j] * cs[j]) + rbf((lo ? -pv[j] : pv[j]) * sn[j]));
-    }
+  for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) ss += __shfl_xor(ss, o);
+  const float r = rsqrtf(ss / (float)D + eps);
+  const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+  float o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = rbf((x[j] * r) * wv[j]);
+  float cs[8], sn[8];
+  unpack8(ca, cs);
+  unpack8(sa, sn);
+  const bool lo = d0 < RD / 2;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float pv = __shfl_xor(x[j], RD / 16);  // every lane of the half wave takes part
+    o[j] = rot ? rbf(rbf(x[j] * cs[j]) + rbf((lo ? -pv : pv) * sn[j])) : x[j];
   }
   uint16_t* dst = isq ? qt + ((int64_t)t * N + n) * D : kt + ((int64_t)(t - HQ) * N + n) * D;
-  *reinterpret_cast<uint2*>(dst + d0) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+  store_nt(dst + d0, make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7])));
 }
 
 hipError_t launch_fullattn_prep(const uint16_t* proj, int64_t N, int HQ, int HKV, int RD, float eps,
                                 const float* qw1, const float* kw1, const uint16_t* cosb, const uint16_t* sinb,
                                 uint16_t* qt, uint16_t* kt, uint16_t* vt, uint16_t* gate, hipStream_t st) {
-  const int64_t G = (HQ + 2 * HKV + 3) / 4;
+  const int64_t G = (HQ + 2 * HKV + 7) / 8;
   hipLaunchKernelGGL(fullattn_prep_k, dim3((unsigned)(N * G)), dim3(256), 0, st, proj, N, HQ, HKV, RD, eps, qw1, kw1,
                      cosb, sinb, qt, kt, vt, gate);
   return hipGetLastError();
@@ -142,10 +145,6 @@ hipError_t launch_fullattn_prep(const uint16_t* proj, int64_t N, int HQ, int HKV
 // 20 KB of each slot go out at about the same time). Graph replays on MI355X, earlier kernel -> this one, and the
 // algorithmic rate: 200 shared rows x 8 paths 16.3 -> 9.8 us (4.4 TB/s), 480 x 8 25.8 -> 18.4, 40 x 4 9.8 -> 4.6,
 // 1600 x 3 42.0 -> 30.4, 1500 x 16 124.4 -> 85-98 us (5.5-6.4 TB/s; a fill reaches 6.9).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store_nt(uint16_t* dst, uint4 v) {
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(dst));
-}
 constexpr int kLinRows = 4;      // rows (waves) per workgroup
 constexpr int kPadGroups = 256;  // padding slots written at a time
 
