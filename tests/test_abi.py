@@ -92,6 +92,21 @@ def test_plan_rule_off_the_table(pkg):
                 assert c.splitk == 1, what
 
 
+def test_plan_rule_is_a_function_of_its_arguments(pkg):
+    """The rule's plans come through a small table per thread: the same sizes in another order, with others in
+    between and from another thread, give the same plans."""
+    import threading
+    args = [(M, N, K, k) for M in (33, 100, 515, 3000) for N in (512, 4096, 5120) for K in (1024, 4160)
+            for k in _plan_kinds(N, K)]
+    ask = lambda a: (lambda c: (c.tile, c.splitk, c.one_launch, c.tail_rows))(pkg._lib.plan(*a))  # noqa: E731
+    first = {a: ask(a) for a in args}
+    got = {}
+    t = threading.Thread(target=lambda: got.update({a: ask(a) for a in args[::-1]}))
+    t.start()
+    t.join()
+    assert got == first and all(ask(a) == first[a] for a in args[::3] + args[::2])
+
+
 def test_plan_table_ranges(pkg):
     """Range rows (m_lo > 0): ordered, disjoint per shape and kind, two-launch, and the plan of every row count in
     them; a row for a single count inside a range goes first."""
