@@ -414,7 +414,8 @@ __device__ __forceinline__ void sk_body(const GemmParams& p) {
 // one kernel that branches between six bodies, over the plans of gate-up, QKV and down at M = 64-2048: 256 x 128 1.3%,
 // 256 x 96 1%, 192 x 288 and 256 x 256 0.5% faster, the others level.
 template <int FN, int FM, int WN, int WM, int EPI, bool PK>
-__global__ void __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm_sk_kernel(const GemmParams p, const int) {
+__global__ void __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_sk_kernel(const GemmParams p, const int) {
   sk_body<FN, FM, WN, WM, EPI, PK>(p);
 }
 
