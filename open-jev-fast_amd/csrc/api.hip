@@ -116,6 +116,13 @@ bool part_fits(int64_t K, int32_t tile, int32_t splitk) {
   return (splitk - 1) * ch < K;  // every split owns a non-empty K range
 }
 
+// The tiles address their operands with 32-bit offsets from the first row of the tile, through descriptors of at most
+// 2^31 - 1 bytes: rows further away would read as zeros.
+bool rows_in_reach(int32_t tile, int64_t M, int64_t N, int64_t ldx, int64_t ldw) {
+  const ojx::TileInfo* t = ojx::tile_info(tile);
+  return std::max(std::min<int64_t>(t->bm, M) * ldx, std::min<int64_t>(t->bn, N) * ldw) * 2 < (1LL << 31);
+}
+
 // Tile families that read the packed layout (without tails, with splits of whole 64-k stages): 0 (both operands
 // through registers and LDS), 5 (persistent) and 6 (K-interleaved).
 bool reads_packed(int32_t tile) {
@@ -248,6 +255,7 @@ ojx_cfg rule_plan(int64_t M, int64_t N, int64_t K, int32_t kind, int32_t planes 
   bool found = false;
   for (const StageCost& sc : kStageCost) {
     const ojx::TileInfo* t = ojx::tile_info(sc.tile);
+    if (!rows_in_reach(sc.tile, M, N, K, K)) continue;  // none left (K in the millions): the small tile of `best`
     const int64_t tiles = cdiv(N, t->bn) * cdiv(M, t->bm), rem = tiles % kPlanCus;
     for (int32_t S : kRuleSplits) {
       if (planes > 0) {
@@ -545,6 +553,7 @@ int ojx_gemm_splitk_f32(const void* x, const void* w, float* parts, int64_t M, i
   if (tile < 0) {
     OJX_TRY(ojx_plan(M, N, K, OJX_KIND_RESIDUAL, &c));
     if (is_sk(c.tile)) c = rule_plan(M, N, K, OJX_KIND_RESIDUAL, S);  // that family writes no K planes
+    if (!rows_in_reach(c.tile, M, N, ldx, ldw)) c.tile = 0;
   } else {
     c.tile = tile;
   }
@@ -570,6 +579,8 @@ static int gemm_bf16_impl(const void* x, const void* w, void* y, int64_t M, int6
     return fail(OJX_ERR_ARG, "y must be 8-byte aligned with row stride >= N and a multiple of 4");
   ojx_cfg c{};
   OJX_TRY(resolve(M, N, K, OJX_KIND_PLAIN | (packed ? OJX_KIND_PACKED : 0), cfg, &c));
+  // the plan knows the sizes, not the row strides; the smallest tile reaches furthest and needs no workspace
+  if (cfg == nullptr && !rows_in_reach(c.tile, M, N, ldx, packed ? K : ldw)) c = ojx_cfg{0, 1, 0, 1, 0, 0};
   OJX_TRY(check_ws(workspace, workspace_bytes, workspace_for(c, M, N, K)));
   hipStream_t st = static_cast<hipStream_t>(stream);
   Part parts[2];

@@ -92,6 +92,15 @@ def test_plan_rule_off_the_table(pkg):
                 assert c.splitk == 1, what
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 64, 1 << 22), (33, 128, 1 << 23), (2048, 1024, 3_500_032), (24, 65536, 1 << 22)])
+@pytest.mark.parametrize("kind", [0, 2])
+def test_plan_rule_keeps_rows_in_reach(pkg, M, N, K, kind):
+    """Tiles address their rows with 32-bit offsets through descriptors of less than 2^31 bytes: a plan's tile rows
+    that exist span no more than that, however long a row is."""
+    t = pkg._lib.tile_info(pkg._lib.plan(M, N, K, kind).tile)
+    assert max(min(t["bm"], M), min(t["bn"], N)) * K * 2 < 2 ** 31, t
+
+
 def test_plan_rule_is_a_function_of_its_arguments(pkg):
     """The rule's plans come through a small table per thread: the same sizes in another order, with others in
     between and from another thread, give the same plans."""

@@ -56,6 +56,29 @@ def test_plain_past_2gib(pkg, ext, O, dev, M, N, K, what):
     torch.cuda.synchronize()
 
 
+def test_rows_far_apart(pkg, O, dev):
+    """x rows 7 million elements apart: the 160 rows of the tile that the sizes alone plan span more than a descriptor's
+    2^31 bytes, so that it may not be used here. Also as fp32 K planes."""
+    lib, check = pkg._lib.lib(), pkg._lib.check
+    M, N, K, ldx, S = 300, 16384, 512, 7_000_064, 2
+    assert pkg._lib.tile_info(pkg._lib.plan(M, N, K, 0).tile)["bm"] * ldx * 2 > GIB2
+    g = torch.Generator(device=dev).manual_seed(5)
+    x = torch.empty((M - 1) * ldx + K, dtype=torch.bfloat16, device=dev).as_strided((M, K), (ldx, 1))
+    x.copy_(torch.randn(M, K, generator=g, device=dev))
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    parts = torch.empty(S, M, N, dtype=torch.float32, device=dev)
+    ws = torch.empty(max(16, lib.ojx_workspace_bytes(M, N, K, 0, None)), dtype=torch.uint8, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    _say(f"case limits strided M={M} N={N} K={K} ldx={ldx}")
+    check(lib.ojx_gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, K, N, ws.data_ptr(), ws.numel(),
+                            None, st))
+    check(lib.ojx_gemm_splitk_f32(x.data_ptr(), w.data_ptr(), parts.data_ptr(), M, N, K, ldx, K, S, -1, st))
+    ref = O.linear_bf16(x.contiguous(), w)
+    _check(O, y, ref, "y")
+    _check(O, parts.sum(0).bfloat16(), ref, "planes")
+
+
 def test_residual_x_past_2gib(pkg, ext, O, dev):
     """The down projection's shape (N = 5120, K = 17408) at M = 65536: x 2.125 GiB, split-K planes past 2 GiB."""
     L = pkg._lib
