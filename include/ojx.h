@@ -88,7 +88,8 @@ int ojx_tile_info(int32_t tile, int32_t* info7);
 
 /* Plan lookup for a shape: a static table measured offline on MI355X (single row counts and ranges of them), and for
  * everything else the (tile, split) with the lowest estimated time.
- * Never times anything, so it is safe during graph capture.
+ * Never times anything, so it is safe during graph capture. N and K of at least 1, M of at least 0 and all below 2^31
+ * (OJX_ERR_SHAPE otherwise, here and, as -1, from ojx_workspace_bytes).
  * Replaces the per-shape cuBLASLt heuristic/search: lt_setup (src/lt.cpp:15-42), _tune (src/fastmodel.py:114-132),
  * lt2_plan / lt2_search (src/lt.cpp:64-159). For OJX_KIND_SILU_MUL, N is the packed 2*I. */
 int ojx_plan(int64_t M, int64_t N, int64_t K, int32_t kind, ojx_cfg* out);
@@ -98,7 +99,7 @@ int ojx_plan(int64_t M, int64_t N, int64_t K, int32_t kind, ojx_cfg* out);
 int ojx_num_candidates(int64_t M, int64_t N, int64_t K, int32_t kind);
 int ojx_candidate(int64_t M, int64_t N, int64_t K, int32_t kind, int32_t idx, ojx_cfg* out);
 
-/* Workspace bytes the call needs with cfg (NULL = the plan's choice). */
+/* Workspace bytes the call needs with cfg (NULL = the plan's choice); -1 with ojx_last_error() set on an error. */
 int64_t ojx_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t kind, const ojx_cfg* cfg);
 
 /* y[M,N] (row stride ldy) = x[M,K] (row stride ldx) . W[N,K]^T (row stride ldw).

@@ -300,8 +300,19 @@ ojx_cfg rule_plan_memo(int64_t M, int64_t N, int64_t K, int32_t kind) {
   return e.c;
 }
 
+// Sizes that a plan or a workspace can be computed for: the arithmetic of both divides by tile counts and K stages.
+int check_sizes(int64_t M, int64_t N, int64_t K) {
+  if (M < 0 || N <= 0 || K <= 0) return fail(OJX_ERR_SHAPE, "bad shape M=%lld N=%lld K=%lld", (long long)M,
+                                              (long long)N, (long long)K);
+  if (M >= (1LL << 31) || N >= (1LL << 31) || K >= (1LL << 31))
+    return fail(OJX_ERR_SHAPE, "shape dimension exceeds 2^31");
+  return OJX_OK;
+}
+
 int resolve(int64_t M, int64_t N, int64_t K, int32_t kind, const ojx_cfg* cfg, ojx_cfg* out) {
   if (cfg != nullptr) {
+    const int rc = check_sizes(M, N, K);
+    if (rc != OJX_OK) return rc;
     if (!cfg_fits(M, N, K, *cfg, is_packed_kind(kind)))
       return fail(OJX_ERR_CONFIG, "config (tile %d, splitk %d, tail %d/%d/%d) invalid for M=%lld N=%lld K=%lld",
                   cfg->tile, cfg->splitk, cfg->tail_tile, cfg->tail_splitk, cfg->tail_rows, (long long)M,
@@ -313,10 +324,8 @@ int resolve(int64_t M, int64_t N, int64_t K, int32_t kind, const ojx_cfg* cfg, o
 }
 
 int check_dims(int64_t M, int64_t N, int64_t K) {
-  if (M < 0 || N <= 0 || K <= 0) return fail(OJX_ERR_SHAPE, "bad shape M=%lld N=%lld K=%lld", (long long)M,
-                                              (long long)N, (long long)K);
-  if (M >= (1LL << 31) || N >= (1LL << 31) || K >= (1LL << 31))
-    return fail(OJX_ERR_SHAPE, "shape dimension exceeds 2^31");
+  const int rc = check_sizes(M, N, K);
+  if (rc != OJX_OK) return rc;
   if (N % 8 != 0 || K % 8 != 0)
     return fail(OJX_ERR_SHAPE, "N (%lld) and K (%lld) must be multiples of 8", (long long)N, (long long)K);
   return OJX_OK;
@@ -489,6 +498,7 @@ int ojx_plan(int64_t M, int64_t N, int64_t K, int32_t kind, ojx_cfg* out) {
   const int32_t base = kind & ~OJX_KIND_PACKED;
   if (base < OJX_KIND_PLAIN || base > OJX_KIND_RESIDUAL || (kind & ~(OJX_KIND_PACKED | 3)) != 0)
     return fail(OJX_ERR_ARG, "unknown kind %d", kind);
+  OJX_TRY(check_sizes(M, N, K));
   const bool packed = is_packed_kind(kind);
   for (const PlanEntry& e : kPlan) {
     if (e.N == N && e.K == K && e.kind == kind && (e.M == M || (e.m_lo > 0 && e.m_lo <= M && M <= e.M))) {

@@ -101,6 +101,35 @@ def test_plan_rule_keeps_rows_in_reach(pkg, M, N, K, kind):
     assert max(min(t["bm"], M), min(t["bn"], N)) * K * 2 < 2 ** 31, t
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2, 4, 5, 6])
+def test_plan_refuses_empty_and_negative_sizes(pkg, kind):
+    """An empty or negative dimension ends in the shape error before any plan arithmetic (which divides by tile
+    counts and K stages), from ojx_plan, ojx_workspace_bytes and the Python entry points' workspace and tuning calls;
+    M = 0 is a plan as before (the launch is then a no-op)."""
+    import torch
+    from importlib import import_module
+    ext = import_module("open_jev_fast_amd.ext")
+    L, c = pkg._lib.lib(), pkg._lib.OjxCfg()
+    given = pkg._lib.cfg(0, 1)
+    bad = [(M, *nk) for M in (0, 7, 24, 64, 300) for b in (0, -8, -64, 1 << 31)
+           for nk in ((b, 5120), (5120, b), (b, b), (b, 64))] + [(-1, 5120, 5120), (-64, 64, 64), (1 << 31, 64, 64)]
+    for M, N, K in bad:
+        assert L.ojx_plan(M, N, K, kind, ctypes.byref(c)) == 2, (M, N, K)
+        assert b"shape" in L.ojx_last_error()
+        for cfg in (None, ctypes.byref(given)):
+            assert L.ojx_workspace_bytes(M, N, K, kind, cfg) == -1, (M, N, K)
+        with pytest.raises(RuntimeError, match="shape"):
+            ext._workspace(M, N, K, kind, None, torch.device("cpu"))
+    assert L.ojx_plan(0, 5120, 5120, kind, ctypes.byref(c)) == 0
+    proj = import_module("open_jev_fast_amd.fastproj").FastProjections()
+    e = lambda *s: torch.empty(*s, dtype=torch.bfloat16)  # noqa: E731
+    for x, w in ((e(64, 0), e(5120, 0)), (e(7, 5120), e(0, 5120))):
+        with pytest.raises(RuntimeError, match="bad shape"):
+            proj._tune(x, w)
+        with pytest.raises(RuntimeError, match="bad shape"):
+            proj._tune_sk(x, w, 2)
+
+
 def test_plan_rule_is_a_function_of_its_arguments(pkg):
     """The rule's plans come through a small table per thread: the same sizes in another order, with others in
     between and from another thread, give the same plans."""

@@ -261,6 +261,18 @@ def test_unsplit_weight_layout(pkg, ext, dev, N, K, S):
         assert ext.unsplit_weight(wsk3) is not u3 and torch.equal(ext.unsplit_weight(wsk3), w * 3)
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 5120, 0), (7, 0, 5120), (300, 0, 0)])
+def test_empty_dimension_raises(ext, dev, M, N, K):
+    """An empty K or N is an error of the call, raised before anything is planned or launched."""
+    _say(f"case empty dimension M={M} N={N} K={K}")
+    x, w = torch.empty(M, K, dtype=torch.bfloat16, device=dev), torch.empty(N, K, dtype=torch.bfloat16, device=dev)
+    h, w1 = torch.empty(M, N, dtype=torch.bfloat16, device=dev), torch.empty(N, device=dev)
+    for call in (lambda: ext.mm(x, w), lambda: ext.mm_silu_mul(x, w),
+                 lambda: ext.mm_residual_rmsnorm(h, x, w, w1, None, 1e-6)):
+        with pytest.raises(RuntimeError, match="shape"):
+            call()
+
+
 # ----------------------------------------------------------------------------------------------- epilogues
 def test_add_rmsnorm_variants(pkg, ext, O, dev):
     M, H = 33, 5120
