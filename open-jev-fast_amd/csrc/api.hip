@@ -117,10 +117,20 @@ bool part_fits(int64_t K, int32_t tile, int32_t splitk) {
 }
 
 // The tiles address their operands with 32-bit offsets from the first row of the tile, through descriptors of at most
-// 2^31 - 1 bytes: rows further away would read as zeros.
-bool rows_in_reach(int32_t tile, int64_t M, int64_t N, int64_t ldx, int64_t ldw) {
+// 2^31 - 1 bytes: rows further away would read as zeros. gemm() refuses such a launch; plans choose around it.
+bool rows_in_reach(int32_t tile, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw) {
   const ojx::TileInfo* t = ojx::tile_info(tile);
-  return std::max(std::min<int64_t>(t->bm, M) * ldx, std::min<int64_t>(t->bn, N) * ldw) * 2 < (1LL << 31);
+  auto reach = [&](int64_t rows, int64_t ld) {  // from the first row's start to the end of the last row's K elements
+    constexpr int64_t kElems = 1LL << 30;
+    return rows <= 1 ? K < kElems : ld < kElems && (rows - 1) * ld + K < kElems;
+  };
+  return reach(std::min<int64_t>(t->bm, M), ldx) && reach(std::min<int64_t>(t->bn, N), ldw);
+}
+
+// The tile for rows that a plan's tile does not reach: of the tiles that read every layout and write every epilogue,
+// one of the two with the fewest rows (64 W rows, 32 W rows; both 16 x rows). Where neither reaches, the launch fails.
+int32_t far_rows_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw) {
+  return rows_in_reach(0, M, N, K, ldx, ldw) ? 0 : 90;
 }
 
 // Tile families that read the packed layout (without tails, with splits of whole 64-k stages): 0 (both operands
@@ -249,13 +259,15 @@ ojx_cfg rule_plan(int64_t M, int64_t N, int64_t K, int32_t kind, int32_t planes 
     const int64_t s = std::min<int64_t>({8, 520 / tiles, K / 512});
     best.splitk = planes > 0 ? planes : (int32_t)std::max<int64_t>(1, residual && N > 8192 ? 1 : s);
     while (planes == 0 && best.splitk > 1 && !cfg_fits(M, N, K, best, packed)) --best.splitk;
+    if (!rows_in_reach(best.tile, M, N, K, K, K))
+      best = ojx_cfg{far_rows_tile(M, N, K, K, K), std::max(planes, 1), 0, 1, 0, 0};
     return best;
   }
   double best_us = 0.0;
   bool found = false;
   for (const StageCost& sc : kStageCost) {
     const ojx::TileInfo* t = ojx::tile_info(sc.tile);
-    if (!rows_in_reach(sc.tile, M, N, K, K)) continue;  // none left (K in the millions): the small tile of `best`
+    if (!rows_in_reach(sc.tile, M, N, K, K, K)) continue;
     const int64_t tiles = cdiv(N, t->bn) * cdiv(M, t->bm), rem = tiles % kPlanCus;
     for (int32_t S : kRuleSplits) {
       if (planes > 0) {
@@ -273,6 +285,7 @@ ojx_cfg rule_plan(int64_t M, int64_t N, int64_t K, int32_t kind, int32_t planes 
       }
     }
   }
+  if (!found) best.tile = far_rows_tile(M, N, K, K, K);  // rows of millions of elements
   if (planes > 0) best.splitk = planes;
   return best;
 }
@@ -340,6 +353,9 @@ int gemm(const ojx_cfg& c, int epi, const void* x, int64_t ldx, const void* w, i
          uint16_t* hn_out = nullptr, bool packed = false, const ojx::FattnParams* fa = nullptr,
          bool equal_chunks = false) {
   const ojx::TileInfo* t = ojx::tile_info(c.tile);
+  if (!rows_in_reach(c.tile, M, N, K, ldx, packed ? K : ldw))
+    return fail(OJX_ERR_SHAPE, "rows of one tile (%d x %d) span 2 GiB or more: K=%lld ldx=%lld ldw=%lld", t->bn, t->bm,
+                (long long)K, (long long)ldx, (long long)ldw);
   ojx::GemmParams p;
   p.fa = fa != nullptr ? *fa : ojx::FattnParams{};
   p.W = static_cast<const uint16_t*>(w);
@@ -563,7 +579,7 @@ int ojx_gemm_splitk_f32(const void* x, const void* w, float* parts, int64_t M, i
   if (tile < 0) {
     OJX_TRY(ojx_plan(M, N, K, OJX_KIND_RESIDUAL, &c));
     if (is_sk(c.tile)) c = rule_plan(M, N, K, OJX_KIND_RESIDUAL, S);  // that family writes no K planes
-    if (!rows_in_reach(c.tile, M, N, ldx, ldw)) c.tile = 0;
+    if (!rows_in_reach(c.tile, M, N, K, ldx, ldw)) c.tile = far_rows_tile(M, N, K, ldx, ldw);
   } else {
     c.tile = tile;
   }
@@ -589,8 +605,10 @@ static int gemm_bf16_impl(const void* x, const void* w, void* y, int64_t M, int6
     return fail(OJX_ERR_ARG, "y must be 8-byte aligned with row stride >= N and a multiple of 4");
   ojx_cfg c{};
   OJX_TRY(resolve(M, N, K, OJX_KIND_PLAIN | (packed ? OJX_KIND_PACKED : 0), cfg, &c));
-  // the plan knows the sizes, not the row strides; the smallest tile reaches furthest and needs no workspace
-  if (cfg == nullptr && !rows_in_reach(c.tile, M, N, ldx, packed ? K : ldw)) c = ojx_cfg{0, 1, 0, 1, 0, 0};
+  // the plan knows the sizes, not the row strides; the small tiles unsplit need no workspace
+  const int64_t ldwr = packed ? K : ldw;
+  if (cfg == nullptr && !rows_in_reach(c.tile, M, N, K, ldx, ldwr))
+    c = ojx_cfg{far_rows_tile(M, N, K, ldx, ldwr), 1, 0, 1, 0, 0};
   OJX_TRY(check_ws(workspace, workspace_bytes, workspace_for(c, M, N, K)));
   hipStream_t st = static_cast<hipStream_t>(stream);
   Part parts[2];

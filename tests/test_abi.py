@@ -92,7 +92,9 @@ def test_plan_rule_off_the_table(pkg):
                 assert c.splitk == 1, what
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 64, 1 << 22), (33, 128, 1 << 23), (2048, 1024, 3_500_032), (24, 65536, 1 << 22)])
+# 64-row tiles reach to K = 2^24, 32-row tiles to 2^25
+@pytest.mark.parametrize("M,N,K", [(300, 64, 1 << 22), (33, 128, 1 << 23), (2048, 1024, 3_500_032), (24, 65536, 1 << 22),
+                                   (24, 64, 20_000_000), (300, 64, (1 << 25) - 64), (16, 8, 1 << 25)])
 @pytest.mark.parametrize("kind", [0, 2])
 def test_plan_rule_keeps_rows_in_reach(pkg, M, N, K, kind):
     """Tiles address their rows with 32-bit offsets through descriptors of less than 2^31 bytes: a plan's tile rows
@@ -128,6 +130,45 @@ def test_plan_refuses_empty_and_negative_sizes(pkg, kind):
             proj._tune(x, w)
         with pytest.raises(RuntimeError, match="bad shape"):
             proj._tune_sk(x, w, 2)
+
+
+def test_rows_out_of_reach_are_refused_before_a_launch(pkg):
+    """Where no tile reaches the rows of the call (or the given one does not), every entry point returns the shape
+    error instead of multiplying zeros: planned and explicit configurations, splits, strides, one-launch, planes, the
+    fused prep. The sizes below the limits pass the same check and end at the launch, so this needs a machine without
+    a GPU (the buffers are host memory)."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("hands host buffers to launches that must fail for want of a GPU")
+    L = pkg._lib.lib()
+    buf = ctypes.create_string_buffer(1 << 12)
+    p = ctypes.cast(ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 16, ctypes.c_void_p)
+    f = ctypes.cast(p, ctypes.POINTER(ctypes.c_float))
+    ws = 1 << 62
+    cfgp = lambda c: None if c is None else ctypes.byref(pkg._lib.cfg(*c))  # noqa: E731
+
+    def refused(rc):
+        assert rc == 2 and b"2 GiB" in L.ojx_last_error(), (rc, L.ojx_last_error())
+
+    def in_reach(rc):  # passes the check: what fails is the launch, for want of a GPU
+        assert rc == 5 and b"2 GiB" not in L.ojx_last_error(), (rc, L.ojx_last_error())
+
+    for M, N, K in ((24, 128, 1 << 25), (300, 64, 1 << 25), (16, 1024, 1 << 25), (1, 64, 1 << 26), (1, 8, 1 << 30)):
+        for c in (None, (0, 1), (90, 2), (73, 4), (80, 3), (0, 2, 0, 1, 0, 1)):
+            refused(L.ojx_gemm_bf16(p, p, p, M, N, K, K, K, N, p, ws, cfgp(c), None))
+            refused(L.ojx_gemm_silu_mul(p, p, p, M, N // 2, K, p, ws, cfgp(c), None))
+            refused(L.ojx_gemm_residual_rmsnorm(p, p, p, p, None, 1e-6, p, p, M, N, K, p, ws, cfgp(c), None))
+        for tile in (-1, 0, 80):
+            refused(L.ojx_gemm_splitk_f32(p, p, p, M, N, K, K, K, 2, tile, None))
+    refused(L.ojx_gemm_qkv_fullattn_prep(p, p, 0, f, f, p, p, p, p, p, p, 4, 1 << 24, 2, 1, 256, 64, 1e-6, None))
+    for ld in ((1 << 30) + 8, 1 << 40, 1 << 62):  # row strides: two rows or more
+        refused(L.ojx_gemm_bf16(p, p, p, 2, 64, 64, ld, 64, 64, p, ws, None, None))
+        refused(L.ojx_gemm_bf16(p, p, p, 1, 64, 64, 64, ld, 64, p, ws, None, None))
+        refused(L.ojx_gemm_splitk_f32(p, p, p, 2, 64, 64, ld, 64, 1, -1, None))
+        refused(L.ojx_gemm_bf16_pk(p, p, p, 2, 64, 64, ld, 64, p, ws, None, None))
+    in_reach(L.ojx_gemm_bf16(p, p, p, 1, 64, 64, 1 << 40, 64, 64, p, ws, None, None))  # one row: its stride is not used
+    in_reach(L.ojx_gemm_bf16(p, p, p, 2, 64, 64, (1 << 30) - 64 - 8, 64, 64, p, ws, None, None))
+    in_reach(L.ojx_gemm_bf16(p, p, p, 24, 64, 20_000_000, 20_000_000, 20_000_000, 64, p, ws, None, None))
 
 
 def test_plan_rule_is_a_function_of_its_arguments(pkg):

@@ -79,6 +79,29 @@ def test_rows_far_apart(pkg, O, dev):
     _check(O, parts.sum(0).bfloat16(), ref, "planes")
 
 
+@pytest.mark.parametrize("kind", ["plain", "residual"])
+def test_rows_of_millions(pkg, ext, O, dev, kind):
+    """Rows of 20 million elements: 64 of them span more than a descriptor's 2^31 bytes, so that the plan takes a tile
+    of 32 W rows. (fp32 sums of 2e7 terms of a unit result: random rounding of about 3e-5, below bf16's 4e-3.)"""
+    M, N, K = 24, 64, 20_000_000
+    _say(f"case limits long rows {kind} M={M} N={N} K={K} plan={pkg._lib.plan(M, N, K, 2 if kind == 'residual' else 0)}")
+    g = torch.Generator(device=dev).manual_seed(11)
+    x = torch.randn(M, K, generator=g, device=dev, dtype=torch.bfloat16)
+    w = torch.randn(N, K, generator=g, device=dev, dtype=torch.bfloat16).mul_(K ** -0.5)
+    ref = torch.zeros(M, N, dtype=torch.float64, device=dev)
+    for k in range(0, K, 1 << 20):
+        ref += (x[:, k:k + (1 << 20)].float() @ w[:, k:k + (1 << 20)].float().t()).double()
+    ref = ref.bfloat16()
+    if kind == "plain":
+        _check(O, ext.mm(x, w), ref, "y")
+        return
+    res, w1 = torch.randn(M, N, generator=g, device=dev).bfloat16(), torch.ones(N, device=dev)
+    h, hn = ext.mm_residual_rmsnorm(res, x, w, w1, None, 1e-6)
+    rh, rhn = ext.add_rmsnorm(res, ref, w1, None, 1e-6)
+    _check(O, h, rh, "h")
+    _check(O, hn, rhn, "hn")
+
+
 def test_residual_x_past_2gib(pkg, ext, O, dev):
     """The down projection's shape (N = 5120, K = 17408) at M = 65536: x 2.125 GiB, split-K planes past 2 GiB."""
     L = pkg._lib
