@@ -110,8 +110,8 @@ __global__ void __launch_bounds__(64 * WN * WM) gemm_nt_kernel(const GemmParams 
   // ojx_pack_weight) goes through one descriptor over the whole buffer, rows past N skipped.
   const bool wpk = p.wpk != 0;
   const __amdgpu_buffer_rsrc_t rsW = wpk ? make_rsrc(p.W, (int64_t)p.N * p.K * 2)
-                                         : make_rsrc(p.W + (int64_t)n0 * p.ldw, (int64_t)min(BN, p.N - n0) * p.ldw * 2);
-  const __amdgpu_buffer_rsrc_t rsX = make_rsrc(p.X + (int64_t)m0 * p.ldx, (int64_t)min(BM, p.M - m0) * p.ldx * 2);
+                                         : make_rows_rsrc(p.W + (int64_t)n0 * p.ldw, min(BN, p.N - n0), p.ldw, p.K);
+  const __amdgpu_buffer_rsrc_t rsX = make_rows_rsrc(p.X + (int64_t)m0 * p.ldx, min(BM, p.M - m0), p.ldx, p.K);
   const int nbw = p.N >> 4;
   uint4 rw[CW], rx[CX];
   auto gload = [&](int k0) {

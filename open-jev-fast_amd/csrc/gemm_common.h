@@ -15,6 +15,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, in
   const int32_t n = bytes > 0x7fffffffLL ? 0x7fffffff : (int32_t)(bytes < 0 ? 0 : bytes);
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, 0x00020000);
 }
+// The descriptor of `rows` rows, stride ld, of which the first K elements are read. It ends with the last row's
+// elements: an offset past them reads zeros also where rows of the tile that do not exist wrap around 2^32 and come
+// back below rows * ld, in a strided operand beyond its last row's end.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rows_rsrc(const uint16_t* base, int rows, int64_t ld, int K) {
+  return make_rsrc(base, ((int64_t)(rows - 1) * ld + K) * 2);
+}
 __device__ __forceinline__ uint4 bload(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }

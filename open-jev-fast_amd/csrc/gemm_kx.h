@@ -191,9 +191,9 @@ __device__ __forceinline__ void kx_body(const GemmParams& p) {
 
   // row-major W: this tile's rows only (rows past N read zeros); packed W: the whole buffer, blocks past N skipped
   const __amdgpu_buffer_rsrc_t rsW = PK ? make_rsrc(p.W, (int64_t)p.N * p.K * 2)
-                                           : make_rsrc(p.W + (int64_t)n0 * p.ldw, (int64_t)min(BN, p.N - n0) * p.ldw * 2);
+                                           : make_rows_rsrc(p.W + (int64_t)n0 * p.ldw, min(BN, p.N - n0), p.ldw, p.K);
   const int nbw = p.N >> 4;  // 16-row blocks of the packed W
-  const __amdgpu_buffer_rsrc_t rsX = make_rsrc(p.X + (int64_t)m0 * p.ldx, (int64_t)min(BM, p.M - m0) * p.ldx * 2);
+  const __amdgpu_buffer_rsrc_t rsX = make_rows_rsrc(p.X + (int64_t)m0 * p.ldx, min(BM, p.M - m0), p.ldx, p.K);
 
   // ------------------------------------------------------------------ fragment ownership
   // extra fragments: x fragment xe, W fragments wstart .. wstart + EW - 1 (walked first)

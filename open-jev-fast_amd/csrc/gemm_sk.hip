@@ -181,8 +181,8 @@ __device__ __forceinline__ void sk_body(const GemmParams& p) {
     // [K/64][N/16][16][64], see ojx_pack_weight) is addressed through one descriptor over the whole buffer: W block
     // blk of a stage is 1 KiB at row block n0/16 + blk/2, half blk & 1, and blocks past N are skipped.
     const __amdgpu_buffer_rsrc_t rsW = PK ? make_rsrc(Wp, (int64_t)N * K * 2)
-                                           : make_rsrc(Wp + (int64_t)n0 * ldw, (int64_t)min(BN, N - n0) * ldw * 2);
-    const __amdgpu_buffer_rsrc_t rsX = make_rsrc(Xp + (int64_t)m0 * ldx, (int64_t)min(BM, M - m0) * ldx * 2);
+                                           : make_rows_rsrc(Wp + (int64_t)n0 * ldw, min(BN, N - n0), ldw, K);
+    const __amdgpu_buffer_rsrc_t rsX = make_rows_rsrc(Xp + (int64_t)m0 * ldx, min(BM, M - m0), ldx, K);
     const __amdgpu_buffer_rsrc_t rsNone = make_rsrc(Wp, 0);
     const uint32_t dWp0 = (uint32_t)((((n0 >> 4) + (wave >> 1)) * 16 + (wave & 1) * 8 + (lane >> 3)) * 128 + kcol * 2);
 

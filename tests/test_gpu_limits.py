@@ -7,6 +7,8 @@ candidate list, and every element is compared with the oracle's arithmetic on th
 within the north star's tolerance. (Packed weights are limited to 2 GiB by ojx_pack_weight; that limit is an
 error-path check here.)
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -77,6 +79,27 @@ def test_rows_far_apart(pkg, O, dev):
     ref = O.linear_bf16(x.contiguous(), w)
     _check(O, y, ref, "y")
     _check(O, parts.sum(0).bfloat16(), ref, "planes")
+
+
+@pytest.mark.parametrize("tile", [0, 87, 104])
+@pytest.mark.parametrize("M", [1, 3])
+def test_absent_rows_wrap_inside_the_operand(pkg, O, dev, M, tile):
+    """Row strides at which the offsets of the tile's absent rows (M .. 15 at least) wrap around 2^32 to between the rows
+    that exist and, for one row, past its end: those lanes must read nothing there. One case per tile family."""
+    lib, check = pkg._lib.lib(), pkg._lib.check
+    N, K = 128, 512
+    ldx = (1 << 28) + (1 << 19) if M > 1 else (1 << 29) - (1 << 19)   # elements: 8 rows are 2^32 bytes and 8 MiB more / less
+    assert any(K * 2 <= m * ldx * 2 % (1 << 32) < ldx * 2 for m in range(M, 16))
+    _say(f"case limits absent rows M={M} tile={tile} ldx={ldx}")
+    g = torch.Generator(device=dev).manual_seed(6)
+    x = torch.empty((M - 1) * ldx + K, dtype=torch.bfloat16, device=dev).as_strided((M, K), (ldx, 1))
+    x.copy_(torch.randn(M, K, generator=g, device=dev))
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    cfg = pkg._lib.cfg(tile, 1)
+    check(lib.ojx_gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, K, N, None, 0, ctypes.byref(cfg),
+                            torch.cuda.current_stream().cuda_stream))
+    _check(O, y, O.linear_bf16(x.contiguous(), w), "y")
 
 
 @pytest.mark.parametrize("kind", ["plain", "residual"])
