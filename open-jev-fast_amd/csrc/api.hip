@@ -790,7 +790,8 @@ static int check_fattn(int64_t N, int32_t HQ, int32_t HKV, int32_t D, int32_t RD
   if (HQ < 1 || HKV < 1 || HQ > 4096 || HKV > 4096) return fail(OJX_ERR_SHAPE, "bad head counts HQ=%d HKV=%d", HQ, HKV);
   if (RD < 16 || RD > D || RD % 16 != 0 || ((RD / 16) & (RD / 16 - 1)) != 0)
     return fail(OJX_ERR_SHAPE, "rotary dims RD=%d must be 16 * a power of two, <= D", RD);
-  if (N < 0 || N * ((HQ + 2 * HKV + 3) / 4) >= (1LL << 31)) return fail(OJX_ERR_SHAPE, "bad token count");
+  if (N < 0 || N >= (1LL << 31) || N * ((HQ + 2 * HKV + 7) / 8) >= (1LL << 31))  // workgroups of eight head tasks
+    return fail(OJX_ERR_SHAPE, "bad token count");
   if (N == 0) return OJX_OK;  // nothing is read or written
   const void* ptrs[] = {qw1, kw1, cosb, sinb, qt, kt, vt, gate};
   for (const void* q : ptrs)
@@ -835,7 +836,7 @@ int ojx_linattn_prep(const void* proj, const int32_t* hist, const int32_t* rep_p
                      int32_t KD, int32_t VD, int32_t HV, int32_t HK, int32_t HD, int32_t rep_qk, void* q, void* k,
                      void* v, float* g, void* beta, ojx_stream_t stream) {
   if (HD != 128) return fail(OJX_ERR_SHAPE, "linear-attention prep supports head_dim 128 (HD=%d)", HD);
-  if (HK < 1 || HK * HD != KD) return fail(OJX_ERR_SHAPE, "KD=%d must be HK * HD (HK=%d)", KD, HK);
+  if (HK < 1 || (int64_t)HK * HD != KD) return fail(OJX_ERR_SHAPE, "KD=%d must be HK * HD (HK=%d)", KD, HK);
   if (HV < 1 || HV > 256 || VD < 8 || VD % 8 != 0)
     return fail(OJX_ERR_SHAPE, "bad value dims VD=%d HV=%d (HV <= 256, VD a multiple of 8)", VD, HV);
   const int rq = rep_qk ? HV / HK : 1;
@@ -843,8 +844,8 @@ int ojx_linattn_prep(const void* proj, const int32_t* hist, const int32_t* rep_p
   if (N < 0 || N >= (1LL << 31) - 1 || R < 0 || R >= (1LL << 31) || L2 < 1 || R % L2 != 0)
     return fail(OJX_ERR_SHAPE, "bad sizes N=%lld R=%lld L2=%lld (R a multiple of L2)", (long long)N, (long long)R,
                 (long long)L2);
-  if (2 * KD + VD > 28672)  // the finished row is held in LDS (2 bytes per conv channel)
-    return fail(OJX_ERR_SHAPE, "2 KD + VD = %d conv channels exceed 28672", 2 * KD + VD);
+  if (3LL * KD + VD >= (1LL << 30))  // the kernel's channel indexes are 32-bit, of a replicated head's row too
+    return fail(OJX_ERR_SHAPE, "KD=%d VD=%d: too many channels", KD, VD);
   if (R == 0) return OJX_OK;
   const void* ptrs[] = {proj, hist, rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta};
   for (const void* p : ptrs)

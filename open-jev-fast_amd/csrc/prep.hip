@@ -3,6 +3,8 @@
 // and writes out by itself, with whole 8- or 16-byte vector stores.
 #include "ojx_internal.h"
 
+#include <algorithm>
+
 namespace ojx {
 
 namespace {
@@ -165,7 +167,8 @@ __global__ void __launch_bounds__(64 * kLinRows) linattn_prep_k(
     const uint16_t* __restrict__ proj, const int4* __restrict__ hist, const int* __restrict__ rep_ptr,
     const int* __restrict__ rep_pos, const uint16_t* __restrict__ convw, const uint16_t* __restrict__ A_log,
     const uint16_t* __restrict__ dt_bias, uint16_t* __restrict__ q, uint16_t* __restrict__ k,
-    uint16_t* __restrict__ v, float* __restrict__ g, uint16_t* __restrict__ beta, int N, int KD, int VD, int HV) {
+    uint16_t* __restrict__ v, float* __restrict__ g, uint16_t* __restrict__ beta, int N, int KD, int VD, int HV,
+    int rg0) {
   constexpr int HD = 128;
   const int C = 2 * KD + VD;
   const int64_t P = (int64_t)C + VD + 2 * HV;
@@ -173,7 +176,7 @@ __global__ void __launch_bounds__(64 * kLinRows) linattn_prep_k(
   const int rb = (N + kLinRows - 1) / kLinRows;  // row groups; padding groups follow
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int T = (C / 8 + 63) / 64 + 1;           // channel blocks of a row, the gates last
-  const int rg = blockIdx.x / T, cb = blockIdx.x - rg * T;
+  const int rgl = blockIdx.x / T, cb = blockIdx.x - rgl * T, rg = rg0 + rgl;  // this launch starts at row group rg0
   const bool pad = rg >= rb;
   const int n = pad ? N : rg * kLinRows + wave;
   if (n >= N && !pad) return;
@@ -268,14 +271,18 @@ hipError_t launch_linattn_prep(const uint16_t* proj, const int32_t* hist, const 
                                const uint16_t* A_log, const uint16_t* dt_bias, int KD, int VD, int HV, int RQ,
                                uint16_t* q, uint16_t* k, uint16_t* v, float* g, uint16_t* beta, hipStream_t st) {
   const int C = 2 * KD + VD;
-  const dim3 grid((unsigned)(((N + kLinRows - 1) / kLinRows + kPadGroups / kLinRows) * ((C / 8 + 63) / 64 + 1)));
-#define OJX_LIN(RQV)                                                                                                 \
-  hipLaunchKernelGGL(linattn_prep_k<RQV>, grid, dim3(64 * kLinRows), 0, st, proj, reinterpret_cast<const int4*>(hist), \
-                     rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta, (int)N, KD, VD, HV)
-  if (RQ == 3) OJX_LIN(3);
-  else OJX_LIN(1);
-#undef OJX_LIN
-  return hipGetLastError();
+  const int64_t T = (C / 8 + 63) / 64 + 1, groups = (N + kLinRows - 1) / kLinRows + kPadGroups / kLinRows;
+  const auto kernel = RQ == 3 ? linattn_prep_k<3> : linattn_prep_k<1>;
+  // A launch has fewer than 2^32 threads: row groups beyond that (rows in the millions) go in further launches.
+  const int64_t per = ((1LL << 32) - 1) / (64 * kLinRows * T);
+  for (int64_t g0 = 0; g0 < groups; g0 += per) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(std::min(per, groups - g0) * T)), dim3(64 * kLinRows), 0, st, proj,
+                       reinterpret_cast<const int4*>(hist), rep_ptr, rep_pos, convw, A_log, dt_bias, q, k, v, g, beta,
+                       (int)N, KD, VD, HV, (int)g0);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
 }
 
 }  // namespace ojx

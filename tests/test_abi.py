@@ -321,6 +321,24 @@ def test_prep_argument_validation_without_gpu(pkg):
     assert la(5, 0, 16, 256, 768, 6, 2, 128, 0, proj=None) == 0             # no slots: nothing to do
 
 
+def test_linattn_prep_channel_limits(pkg):
+    """Channel counts past the 28672 that an earlier kernel held in LDS pass the checks (and end at the launch, for
+    want of a GPU); sizes whose products leave 32 bits are refused."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("hands host buffers to launches that must fail for want of a GPU")
+    L = pkg._lib.lib()
+    buf = ctypes.create_string_buffer(1 << 12)
+    p = ctypes.cast(ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 16, ctypes.c_void_p)
+    f = ctypes.cast(p, ctypes.POINTER(ctypes.c_float))
+    la = lambda KD, VD, HK, N=5: L.ojx_linattn_prep(p, p, p, p, N, 32, 16, p, p, p, KD, VD, 6, HK, 128, 0, p, p,  # noqa: E731
+                                                    p, f, p, None)
+    assert la(256, 28160, 2) == 5 and la(256, 28168, 2) == 5 and la(16384, 32768, 128) == 5
+    assert la(256, 768, 2, N=1 << 24) == 5
+    assert la(0, 768, 1 << 25) == 2 and la(128, 768, (1 << 25) + 1) == 2   # HK HD wraps to KD in 32 bits
+    assert la(1 << 30, 768, 1 << 23) == 2 and la(256, (1 << 31) - 8, 2) == 2
+
+
 def test_python_mirror_errors_without_gpu(pkg):
     import torch
     from importlib import import_module

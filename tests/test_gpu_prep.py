@@ -214,6 +214,61 @@ def test_linattn_prep_many_slots(ext, dev, Lr, paths, short, HK, HV, PB, rep_qk)
     assert all(bool((t.cpu()[pad] == 0).all()) for t in got)
 
 
+def test_linattn_prep_wide_rows(ext, dev):
+    """64 q/k heads and 20480 value channels: 36864 conv channels, 72 channel blocks a row."""
+    _say("case linattn_prep wide rows")
+    LO, lay, proj, convw, A_log, dt_bias, KD, VD = _lin_inputs((9, [2], [0, 0], [3, 4]), 64, 160, seed=5, NB=1, PB=8)
+    d = lambda a: torch.as_tensor(a).to(dev).contiguous()  # noqa: E731
+    args = (lay["hist"], lay["rep_ptr"], lay["rep_pos"])
+    got = ext.linattn_prep_dedup2(proj.to(dev), *map(d, args), lay["L2"], convw.to(dev), A_log.to(dev),
+                                  dt_bias.to(dev), KD, VD, 160, 64, 128, False)
+    want = LO.linattn_prep(proj, *args, lay["L2"], convw, A_log, dt_bias, KD, VD, 160, 64, 128, False)
+    for o, r, nm, steps in zip(got, want, "q k v g beta".split(), (2, 2, 1, 0, 1)):
+        if nm == "g":
+            assert torch.allclose(o.cpu(), r, rtol=2e-6, atol=0)
+        else:
+            _ulp_close(o, r, nm, min_equal=0.98, steps=steps)
+
+
+def test_linattn_prep_more_rows_than_a_launch(ext, dev):
+    """33.6 million packed rows of the smallest width: their row groups take two launches. Rows at both ends and around
+    the cut hold one slot each (no history), the others none; the padding slots belong to the second launch."""
+    from oracle import linattn_oracle as LO
+    KD, VD, HV, HK = 128, 8, 1, 1
+    C = 2 * KD + VD
+    cut = ((1 << 32) - 1) // (256 * 2) * 4
+    N = cut + 1000
+    rows = [0, 1, 3, cut - 4, cut - 1, cut, cut + 1, cut + 5, N - 1]
+    pads, L2 = 300, 309
+    _say(f"case linattn_prep rows N={N}")
+    g = torch.Generator().manual_seed(12)
+    small = (torch.randn(len(rows), C + VD + 2 * HV, generator=g) * 1.5).bfloat16()
+    convw, A_log, dt_bias = torch.randn(C, 4, generator=g).bfloat16(), torch.randn(HV, generator=g).bfloat16(), \
+        torch.randn(HV, generator=g).bfloat16()
+    at = torch.tensor(rows, device=dev)
+    proj = torch.empty(N, small.shape[1], dtype=torch.bfloat16, device=dev)   # 18 GB, read at `rows` only
+    proj[at] = small.to(dev)
+    hist = torch.full((N + 1, 4), -1, dtype=torch.int32, device=dev)
+    hist[at, 3] = at.int()
+    held = torch.zeros(N + 1, dtype=torch.int32, device=dev)
+    held[at] = 1
+    held[N] = pads
+    rep_ptr = torch.cat([torch.zeros(1, dtype=torch.int32, device=dev), held.cumsum(0).int()])
+    rep_pos = torch.randperm(L2, generator=g).int()
+    got = ext.linattn_prep_dedup2(proj, hist, rep_ptr, rep_pos.to(dev), L2, convw.to(dev), A_log.to(dev),
+                                  dt_bias.to(dev), KD, VD, HV, HK, 128, False)
+    n = len(rows)
+    h = torch.full((n + 1, 4), -1, dtype=torch.int32)
+    h[:n, 3] = torch.arange(n, dtype=torch.int32)
+    want = LO.linattn_prep(small, h.numpy(), list(range(n + 1)) + [n + pads], rep_pos.numpy(), L2, convw, A_log,
+                           dt_bias, KD, VD, HV, HK, 128, False)
+    for o, r, nm, steps in zip(got, want, "q k v g beta".split(), (2, 2, 1, 0, 1)):
+        if nm == "g":
+            assert torch.allclose(o.cpu(), r, rtol=2e-6, atol=0)
+        else:
+            _ulp_close(o, r, nm, min_equal=0.98, steps=steps)
+
+
 def test_linattn_prep_rejects(ext, dev):
     LO, lay, proj, convw, A_log, dt_bias, KD, VD = _lin_inputs(_TREES["nopad"], 2, 6, seed=1)
     d = lambda a: torch.as_tensor(a).to(dev).contiguous()  # noqa: E731
