@@ -171,6 +171,16 @@ def test_rows_out_of_reach_are_refused_before_a_launch(pkg):
     in_reach(L.ojx_gemm_bf16(p, p, p, 24, 64, 20_000_000, 20_000_000, 20_000_000, 64, p, ws, None, None))
 
 
+def test_ragged_cases_reach_every_family(pkg):
+    """The GPU cases with a partial last K stage are planned on the families and splits that they name: split and
+    unsplit tiles of families 0 and 6, persistent tiles with a spread, all three kinds."""
+    from tests.test_gpu_random_shapes import RAGGED_PLANS
+    for kind, M, N, K, family, split in RAGGED_PLANS:
+        c = pkg._lib.plan(M, N, K, ("plain", "silu", "residual").index(kind))
+        got = (pkg._lib.tile_info(c.tile)["family"], c.splitk > 1)
+        assert K % 64 and got == (family, split), (kind, M, N, K, c)
+
+
 def test_plan_rule_is_a_function_of_its_arguments(pkg):
     """The rule's plans come through a small table per thread: the same sizes in another order, with others in
     between and from another thread, give the same plans."""
