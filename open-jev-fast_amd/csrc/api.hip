@@ -201,22 +201,14 @@ int64_t workspace_for(const ojx_cfg& c, int64_t M, int64_t N, int64_t K) {
 }
 
 // The plan of every call that no table row covers: the (tile, split) with the lowest estimated time.
-//
-// Time of one 64-k stage of a tile with the whole chip running it (us). Fitted, with the constants of plan_us, to the
-// candidates within 30% of the best at 49 row counts (1-2048) of eight projection shapes and both weight layouts on
-// MI355X; picking by the estimate costs 2.4% of the best candidate's time on average there (8% at the 90th
-// percentile).
+// The package's planfit.py restates the rule in Python (a test compares the two) and fits its constants.
 struct StageCost {
   int32_t tile;
   double us;
 };
-constexpr StageCost kStageCost[] = {
-    {73, 1.462}, {74, 1.761}, {75, 0.861}, {76, 1.165}, {80, 1.178}, {81, 1.032}, {82, 0.843}, {83, 0.918},
-    {84, 0.498}, {85, 0.729}, {86, 0.650}, {92, 1.143}, {93, 0.714}, {94, 0.489}, {95, 0.531}, {96, 0.718},
-    {97, 0.883}, {98, 0.878}, {99, 0.996}, {100, 1.030}, {101, 1.346}, {102, 1.369}, {103, 0.688}, {104, 0.502}};
+#include "plan_rule.inc"
 constexpr int kRuleSplits[] = {1, 2, 3, 4, 6, 8};
 constexpr int64_t kPlanCus = 256;     // the plan does not depend on the machine that asks for it
-constexpr double kHbmBytesPerUs = 6.63e6;
 
 // Estimated time (us) of an M x N x K projection on tile t in S splits (persistent tiles: stream-K spread S; only
 // spreads that cut every remainder tile into S equal pieces are estimated, uneven ones measured up to 60% slower).
@@ -233,13 +225,14 @@ double plan_us(const ojx::TileInfo* t, double stage, int64_t M, int64_t N, int64
     const int64_t ipt = cdiv(K, 64), full = tiles / kPlanCus, rem = tiles - full * kPlanCus;
     const int64_t gs = std::min(rem * S, rem * ipt);
     const int64_t its = full * ipt + (rem > 0 ? cdiv(rem * ipt, gs) : 0);
-    double us = (double)its * rate(full > 0 ? kPlanCus : gs) + 9.82 * (double)(full + (rem > 0 ? 1 : 0));
-    if (gs > rem) us += (residual ? 0.0 : 5.21) + 2.0 * (double)(gs + rem) * t->bn * t->bm * 4.0 / 14.02e6;
+    double us = (double)its * rate(full > 0 ? kPlanCus : gs) + kTileUs * (double)(full + (rem > 0 ? 1 : 0));
+    if (gs > rem)
+      us += (residual ? 0.0 : kPieceLaunchUs) + 2.0 * (double)(gs + rem) * t->bn * t->bm * 4.0 / kPieceBytesPerUs;
     return us;
   }
   const int64_t nk = cdiv(cdiv(K, S), 64), wgs = tiles * S, rounds = cdiv(wgs, kPlanCus);
-  double us = (double)rounds * ((double)nk * rate(wgs) + 6.59);
-  if (S > 1) us += (residual ? 0.0 : 4.47) + 2.0 * (double)S * (double)M * (double)N * 4.0 / 8.44e6;
+  double us = (double)rounds * ((double)nk * rate(wgs) + kRoundUs);
+  if (S > 1) us += (residual ? 0.0 : kPlaneLaunchUs) + 2.0 * (double)S * (double)M * (double)N * 4.0 / kPlaneBytesPerUs;
   return us;
 }
 

@@ -1,9 +1,14 @@
-"""Offline tuner: measures every (tile, split-K) candidate for the projection shapes on this GPU and writes the
-plan table (csrc/plan_table.inc) that ojx_plan() reads. Replaces the reference's per-shape cuBLASLt searches
+"""Offline tuner: measures every (tile, split-K) candidate for the projection shapes on this GPU and puts the winners
+into the plan table (csrc/plan_table.inc) that ojx_plan() reads. Replaces the reference's per-shape cuBLASLt searches
 (_tune src/fastmodel.py:114-132, bench/lt_search.py) with a one-time offline sweep, so nothing is timed at run
 time or during graph capture.
 
-    python open-jev-fast_amd/tune.py --out /tmp/plan_table.inc [--m 7,288] [--shapes gate_up,down]
+    python open-jev-fast_amd/tune.py --out open-jev-fast_amd/csrc/plan_table.inc [--m 7,288] [--shapes gate_up,down]
+    python open-jev-fast_amd/tune.py --data /tmp/candidates.csv --two-launch --no-tails --m 33,96,... [--packed]
+
+--out replaces the single rows of the measured (shape, M) in that file, adds those it does not have, and keeps every
+other row (ranges of row counts among them) as it is. --data writes every candidate's time: what planfit.py judges and
+fits the plan rule by, and takes range rows from. A range row covers calls that a single row does not.
 
 Each candidate is timed by graph replay over rotating weight copies (larger than the Infinity Cache); the winner
 is checked against a torch fp32 GEMM on the GPU before it is accepted (max rel 1e-2, mean |d| <= 1e-3 RMS).
@@ -11,6 +16,7 @@ is checked against a torch fp32 GEMM on the GPU before it is accepted (max rel 1
 import argparse
 import json
 import os
+import re
 import sys
 
 import torch
@@ -25,10 +31,39 @@ TUNE_SHAPES = {  # name: (N, K, kind); gate-up N is the packed 2 I
     "lin_in_real": (16480, 5120, "plain"),
     "c1_5120": (5120, 5120, "plain"),
     "gate_up": (34816, 5120, "silu"),
+    "gate_up_plain": (34816, 5120, "plain"),
     "down": (5120, 17408, "residual"),
     "o_proj": (5120, 6144, "residual"),
 }
 M_DEFAULT = (1, 7, 16, 64, 128, 288, 539, 1024, 2048)
+
+
+def merge_table(text, rows):
+    """The plan table's text with the single rows (M, N, K, kind, (tile, splitk, tail_tile, tail_splitk, tail_rows,
+    one_launch), seconds) put in place: a row of the same call is replaced, a new one goes after the last single row of
+    its shape and kind (or of the table), every other line stays."""
+    lines = text.splitlines()
+
+    def fields(line):
+        m = re.match(r"\{([^}]*)\}", line)
+        return [int(v) for v in m.group(1).split(",")] if m else None
+
+    for M, N, K, kind, cfg, t in rows:
+        new = f"{{{M}, {N}, {K}, {kind}, {', '.join(str(v) for v in cfg)}, 0}},  // {t * 1e6:.1f} us"
+        at = last = None
+        for i, line in enumerate(lines):
+            f = fields(line)
+            if f is None or (len(f) > 10 and f[10] != 0):
+                continue
+            if f[:4] == [M, N, K, kind]:
+                at = i
+            if last is None or f[1:4] == [N, K, kind] or fields(lines[last])[1:4] != [N, K, kind]:
+                last = i
+        if at is not None:
+            lines[at] = new
+        else:
+            lines.insert(0 if last is None else last + 1, new)
+    return "\n".join(lines) + "\n"
 
 
 def main():
@@ -49,6 +84,10 @@ def main():
     ap.add_argument("--tiles", default="", help="only these tile ids")
     ap.add_argument("--max-waves", type=float, default=16.0, help="skip candidates with more workgroups than this "
                     "many per CU")
+    ap.add_argument("--splits", default="", help="only these split-K counts")
+    ap.add_argument("--two-launch", action="store_true", help="no one-launch candidates")
+    ap.add_argument("--settle", type=float, default=0.05, help="seconds of untimed replays before each candidate")
+    ap.add_argument("--data", default="", help="append every candidate's time to this CSV")
     ap.add_argument("--no-tails", action="store_true", help="simple (tile, split-K) candidates only")
     ap.add_argument("--sk-splits", default="1,2,3,4,6,8", help="stream-K spreads tried for the persistent family")
     ap.add_argument("--packed", action="store_true", help="tune the packed-weight entry points (kind | 4; the "
@@ -57,6 +96,10 @@ def main():
     Ms = [int(m) for m in args.m.split(",")] if args.m else list(M_DEFAULT)
     sk_splits = {int(v) for v in args.sk_splits.split(",")}
     names = args.shapes.split(",") if args.shapes else list(TUNE_SHAPES)
+    splits = {int(v) for v in args.splits.split(",")} if args.splits else None
+    if args.data and not os.path.exists(args.data):
+        with open(args.data, "w") as f:
+            f.write("kind,N,K,M,tile,splitk,one_launch,us\n")
     rows = []
     dev = "cuda"
     for name in names:
@@ -85,14 +128,16 @@ def main():
             def timed(key):
                 try:
                     cc = _lib.cfg(*key)
-                    t = perf.gpu_time([call(w, cc) for w in ws], iters=args.iters, reps=args.reps, settle=0.05)
+                    t = perf.gpu_time([call(w, cc) for w in ws], iters=args.iters, reps=args.reps, settle=args.settle)
                 except RuntimeError as e:
                     print(json.dumps({"shape": name, "M": M, "cfg": key, "error": str(e)}), flush=True)
                     return
                 results.append((t, key))
 
             for c in _lib.candidates(M, N, K, kid):
-                if only is not None and c.tile not in only:
+                if (only is not None and c.tile not in only) or (splits is not None and c.splitk not in splits):
+                    continue
+                if args.two_launch and c.one_launch:
                     continue
                 info = _lib.tile_info(c.tile)
                 if info["family"] == 5:  # persistent: one workgroup per CU; splitk is the stream-K spread
@@ -131,6 +176,11 @@ def main():
                             continue
                         timed((tile, S, c.tile, c.splitk, tr, 0))
             results.sort()
+            if args.data:
+                with open(args.data, "a") as f:
+                    for t, k in results:
+                        if k[4] == 0:
+                            f.write(f"{kid},{N},{K},{M},{k[0]},{k[1]},{k[5]},{t * 1e6:.2f}\n")
             # accept the fastest candidate whose numerics pass
             ref = None
             best = None
@@ -172,11 +222,9 @@ def main():
         del ws, ws_rm
         torch.cuda.empty_cache()
     if args.out:
+        text = open(args.out).read() if os.path.exists(args.out) else ""
         with open(args.out, "w") as f:
-            f.write("// {M, N, K, kind, tile, splitk, tail_tile, tail_splitk, tail_rows, one_launch} measured by "
-                    "open-jev-fast_amd/tune.py on MI355X (us in comment)\n")
-            for M, N, K, kid, key, t in rows:
-                f.write(f"{{{M}, {N}, {K}, {kid}, {', '.join(str(v) for v in key)}}},  // {t * 1e6:.1f} us\n")
+            f.write(merge_table(text, rows))
 
 
 if __name__ == "__main__":

@@ -196,6 +196,61 @@ def test_plan_rule_is_a_function_of_its_arguments(pkg):
     assert got == first and all(ask(a) == first[a] for a in args[::3] + args[::2])
 
 
+def test_planfit_restates_the_rule(pkg, tmp_path):
+    """The Python restatement that judges and fits the rule picks what the library's rule picks, over random calls that
+    no table row covers; its constants file reads back as written."""
+    import random
+    from importlib import import_module
+    fit = import_module("open_jev_fast_amd.planfit")
+    tiles = {t: pkg._lib.tile_info(t) for t in range(pkg._lib.lib().ojx_num_tiles())}
+    rule = fit.read_rule()
+    fit.write_rule(tmp_path / "rule.inc", *rule)
+    assert (tmp_path / "rule.inc").read_text() == open(fit.RULE_INC).read()
+    rng = random.Random(4)
+    for _ in range(600):
+        M, N, K = int(2 ** rng.uniform(4.2, 12)), 8 * rng.randint(4, 5000), 8 * rng.randint(8, 2500)
+        kind = rng.choice([0, 1, 2])
+        c = pkg._lib.plan(M, N, K, kind)
+        pick = fit.rule_pick(tiles, rule, M, N, K, kind)
+        assert pick is None or pick == (c.tile, c.splitk), (M, N, K, kind, c)
+
+
+def test_planfit_costs_and_ranges(pkg):
+    """Costs and range rows from a made-up measured set: the rule's pick is 10% behind one plan at M = 96 and 112 and the
+    best one elsewhere, so that one range row covers 65 (after the measured 64) to 112."""
+    from importlib import import_module
+    fit = import_module("open_jev_fast_amd.planfit")
+    tiles = {t: pkg._lib.tile_info(t) for t in range(pkg._lib.lib().ojx_num_tiles())}
+    rule, N, K = fit.read_rule(), 7168, 4096
+    pts = {}
+    for M in (48, 64, 96, 112, 160):
+        p = fit.rule_pick(tiles, rule, M, N, K, 0)
+        pts[0, N, K, M] = {p: 110.0, (6, 1): 100.0 if M in (96, 112) else 200.0}
+    n, mean, p90, worst, missing = fit.cost_summary(pts, lambda k: fit.rule_pick(tiles, rule, k[3], k[1], k[2], k[0]))
+    assert (n, missing) == (5, 0) and abs(mean - 0.04) < 1e-9 and abs(worst - 0.1) < 1e-9
+    assert fit.ranges(pts, tiles, rule) == [(112, N, K, 0, 6, 1, 65, 100.0)]
+
+
+def test_tuner_keeps_the_rows_it_did_not_measure(pkg):
+    """tune.py --out changes the measured single rows only: ranges, comments and the other rows stay, new calls go to
+    their shape's rows."""
+    from importlib import import_module
+    tune = import_module("open_jev_fast_amd.tune")
+    text = open(os.path.join(os.path.dirname(pkg.__file__), "csrc", "plan_table.inc")).read()
+    assert tune.merge_table(text, []) == text
+    new = tune.merge_table(text, [(288, 34816, 5120, 1, (73, 2, 0, 1, 0, 0), 1e-4), (300, 34816, 5120, 1, (80, 1, 0, 1, 0, 0), 2e-4),
+                                  (5, 512, 512, 0, (0, 1, 0, 1, 0, 0), 3e-6)])
+    old, got = text.splitlines(), new.splitlines()
+    assert len(got) == len(old) + 2
+    assert set(got) - set(old) == {"{288, 34816, 5120, 1, 73, 2, 0, 1, 0, 0, 0},  // 100.0 us",
+                                   "{300, 34816, 5120, 1, 80, 1, 0, 1, 0, 0, 0},  // 200.0 us",
+                                   "{5, 512, 512, 0, 0, 1, 0, 1, 0, 0, 0},  // 3.0 us"}
+    assert [l for l in old if l not in got] == [l for l in old if l.startswith("{288, 34816, 5120, 1,")]
+    assert [l for l in got if l in set(old)] == [l for l in old if l in set(got)]
+    assert got.index("{300, 34816, 5120, 1, 80, 1, 0, 1, 0, 0, 0},  // 200.0 us") < next(
+        i for i, l in enumerate(got) if l.startswith("// ---- ranges"))
+
+
 def test_plan_table_ranges(pkg):
     """Range rows (m_lo > 0): ordered, disjoint per shape and kind, two-launch, and the plan of every row count in
     them; a row for a single count inside a range goes first."""
