@@ -18,10 +18,12 @@ __device__ __forceinline__ void unpack8(uint4 a, float (&v)[8]) {
   }
 }
 
-// Non-temporal store of a lane's 16 bytes: for output lines that are written whole and read by another kernel.
+// Store of a lane's 16 bytes; NT: non-temporal, past the caches.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store_nt(uint16_t* dst, uint4 v) {
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(dst));
+template <bool NT>
+__device__ __forceinline__ void store16(uint16_t* dst, uint4 v) {
+  if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(dst));
+  else *reinterpret_cast<uint4*>(dst) = v;
 }
 
 }  // namespace
@@ -40,12 +42,15 @@ __device__ __forceinline__ void store_nt(uint16_t* dst, uint4 v) {
 // Work layout: half a wave per (token, head task), eight tasks per workgroup. Task t of a token: t < HQ the q head t
 // (the half wave also copies gate head t), HQ <= t < HQ + HKV the k head t - HQ, then the v heads (copies). Lane l of
 // the 32 owns dims 8l .. 8l+7: one 16-byte load and store each, 512 contiguous bytes per head. A q/k head's sum of
-// squares is five shuffles; the rotary partner dims d -+ RD/2 are all held by lane l ^ (RD / 16) (RD is 16 times a power
-// of two), so the exchange is a shuffle of the eight values: no LDS, no barrier.
-// What bounds it: the launch up to a few hundred tokens, then its bytes. Stores are non-temporal (whole lines, read by
-// another kernel). Graph replays over rotating inputs; an earlier kernel (a wave of 8-byte lanes per task, the partner
-// through LDS, plain stores) -> the same with non-temporal stores -> this: M = 288 6.6 -> 6.1 -> 5.4 us, M = 539 9.4 ->
-// 8.6 -> 7.5, M = 1024 15.2 -> 13.5 -> 12.2 (4.8 TB/s), M = 2048 31.1 -> 30.4 -> 23.0 (5.1 TB/s); M = 7 2.7 -> 2.9.
+// squares is five shuffles; the rotary partner dims d -+ RD/2 are all held by lane l ^ (RD / 16) (RD is 16 times a
+// power of two), so the exchange is a shuffle of the eight values: no LDS, no barrier.
+// What bounds it: the launch up to a few hundred tokens, then its bytes. Graph replays over rotating inputs, an
+// earlier kernel (a wave of 8-byte lanes per task, the partner through LDS) -> this one: M = 288 6.5 -> 6.1 us, M =
+// 539 11.4 -> 9.6, M = 1024 17.7 -> 14.9 (4.0 TB/s), M = 2048 31.6 -> 24.2 (4.8 TB/s).
+// Its stores are ordinary ones. Non-temporal stores make the prep itself up to 1.3 us shorter, but the attention's
+// reads then miss the caches: with a kernel that reads the four outputs behind it, M = 7 10.8 -> 11.6 us, M = 539 26.0
+// -> 27.1, M = 1024 31.9 -> 33.9, M = 2048 48.3 -> 54.0; with the projection in front as well M = 288 73.4 -> 73.4, M
+// = 1024 156.0 -> 158.0, M = 2048 301.2 -> 304.3.
 __global__ void __launch_bounds__(256) fullattn_prep_k(const uint16_t* __restrict__ proj, int64_t N, int HQ, int HKV,
                                                        int RD, float eps, const float* __restrict__ qw1,
                                                        const float* __restrict__ kw1, const uint16_t* __restrict__ cosb,
@@ -63,16 +68,16 @@ __global__ void __launch_bounds__(256) fullattn_prep_k(const uint16_t* __restric
   const int d0 = l * 8;
   if (t >= HQ + HKV) {  // v head: a copy into [HKV, N, D]
     const int hv = t - HQ - HKV;
-    store_nt(vt + ((int64_t)hv * N + n) * D + d0,
-             *reinterpret_cast<const uint4*>(row + (int64_t)(2 * HQ + HKV) * D + hv * D + d0));
+    *reinterpret_cast<uint4*>(vt + ((int64_t)hv * N + n) * D + d0) =
+        *reinterpret_cast<const uint4*>(row + (int64_t)(2 * HQ + HKV) * D + hv * D + d0);
     return;
   }
   const bool isq = t < HQ;
   const uint4 xa = *reinterpret_cast<const uint4*>(
       row + (isq ? (int64_t)t * 2 * D : (int64_t)2 * HQ * D + (int64_t)(t - HQ) * D) + d0);
   if (isq)  // gate head: a copy into [N, HQ D]
-    store_nt(gate + n * (int64_t)(HQ * D) + t * D + d0,
-             *reinterpret_cast<const uint4*>(row + (int64_t)t * 2 * D + D + d0));
+    *reinterpret_cast<uint4*>(gate + n * (int64_t)(HQ * D) + t * D + d0) =
+        *reinterpret_cast<const uint4*>(row + (int64_t)t * 2 * D + D + d0);
   const float* w1 = (isq ? qw1 : kw1) + d0;
   const float4 wa = *reinterpret_cast<const float4*>(w1), wb = *reinterpret_cast<const float4*>(w1 + 4);
   const bool rot = d0 < RD;
@@ -103,7 +108,8 @@ __global__ void __launch_bounds__(256) fullattn_prep_k(const uint16_t* __restric
     o[j] = rot ? rbf(rbf(x[j] * cs[j]) + rbf((lo ? -pv : pv) * sn[j])) : x[j];
   }
   uint16_t* dst = isq ? qt + ((int64_t)t * N + n) * D : kt + ((int64_t)(t - HQ) * N + n) * D;
-  store_nt(dst + d0, make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7])));
+  *reinterpret_cast<uint4*>(dst + d0) =
+      make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
 }
 
 hipError_t launch_fullattn_prep(const uint16_t* proj, int64_t N, int HQ, int HKV, int RD, float eps,
@@ -142,13 +148,19 @@ hipError_t launch_fullattn_prep(const uint16_t* proj, int64_t N, int HQ, int HKV
 // block, the last, computes the gates. The row groups after the rows write zeros to the padding slots, kPadGroups
 // slots at a time.
 // What bounds it: the slot rows written, once a tree has a few hundred slots (below that, the launch and one chain of
-// loads). The slot stores are non-temporal: every line is written whole and read by another kernel, and the hint took
-// the largest tree below from 118.4 to 85-98 us (the channel blocks of a row are neighbouring workgroups, so that its
-// 20 KB of each slot go out at about the same time). Graph replays on MI355X, earlier kernel -> this one, and the
-// algorithmic rate: 200 shared rows x 8 paths 16.3 -> 9.8 us (4.4 TB/s), 480 x 8 25.8 -> 18.4, 40 x 4 9.8 -> 4.6,
-// 1600 x 3 42.0 -> 30.4, 1500 x 16 124.4 -> 85-98 us (5.5-6.4 TB/s; a fill reaches 6.9).
+// loads). The channel blocks of a row are neighbouring workgroups, so that its 20 KB of each slot go out at about the
+// same time. Graph replays on MI355X over rotating inputs, earlier kernel -> this one, and the algorithmic rate: 200
+// shared rows x 8 paths 15.8 -> 10.3 us (4.2 TB/s), 480 x 8 26.3 -> 20.6 (4.6 TB/s), 1500 x 16 125.3 -> 99.6 (5.4
+// TB/s).
+// NT, non-temporal slot stores, from 256 MB of outputs on (what the Infinity Cache holds). Below, the next kernel
+// finds much of the slots there after ordinary stores and none of them after non-temporal ones; above, it misses
+// either way and the stores are faster. Prep and a kernel that reads its outputs, ordinary -> non-temporal: 200 x 8
+// (37 MB) 32.8 -> 36.8 us, 480 x 8 (82 MB) 54.8 -> 64.8, 900 x 8 (154 MB) 93.6 -> 107.6, 900 x 12 (231 MB) 150.4 ->
+// 149.7, 900 x 16 (308 MB) 189.7 -> 188.0 (with the projection in front 369.5 -> 359.7), 1500 x 16 (505 MB) 299.2 ->
+// 294.3.
 constexpr int kLinRows = 4;      // rows (waves) per workgroup
 constexpr int kPadGroups = 256;  // padding slots written at a time
+constexpr int64_t kNtBytes = 256LL << 20;  // outputs of this size and more go past the caches
 
 // Calls put(s) for each of the slots rep_pos[p0], rep_pos[p0 + step], ... below p1; sid holds the first 64 of them,
 // one per lane. Every lane of the wave takes part.
@@ -162,7 +174,7 @@ __device__ __forceinline__ void each_slot(const int* __restrict__ rep_pos, int p
   }
 }
 
-template <int RQ>
+template <int RQ, bool NT>
 __global__ void __launch_bounds__(64 * kLinRows) linattn_prep_k(
     const uint16_t* __restrict__ proj, const int4* __restrict__ hist, const int* __restrict__ rep_ptr,
     const int* __restrict__ rep_pos, const uint16_t* __restrict__ convw, const uint16_t* __restrict__ A_log,
@@ -258,10 +270,10 @@ __global__ void __launch_bounds__(64 * kLinRows) linattn_prep_k(
   each_slot(rep_pos, p0, p1, step, sid, [&](int64_t s) {
     if (!live) return;
     uint16_t* const d = dst + s * ld;
-    store_nt(d, val);
+    store16<NT>(d, val);
     if (RQ > 1 && isqk) {
 #pragma unroll
-      for (int r = 1; r < RQ; ++r) store_nt(d + r * HD, val);
+      for (int r = 1; r < RQ; ++r) store16<NT>(d + r * HD, val);
     }
   });
 }
@@ -272,7 +284,9 @@ hipError_t launch_linattn_prep(const uint16_t* proj, const int32_t* hist, const 
                                uint16_t* q, uint16_t* k, uint16_t* v, float* g, uint16_t* beta, hipStream_t st) {
   const int C = 2 * KD + VD;
   const int64_t T = (C / 8 + 63) / 64 + 1, groups = (N + kLinRows - 1) / kLinRows + kPadGroups / kLinRows;
-  const auto kernel = RQ == 3 ? linattn_prep_k<3> : linattn_prep_k<1>;
+  const bool nt = R * (2LL * (2 * RQ * (int64_t)KD + VD) + 6LL * HV) >= kNtBytes;
+  const auto kernel = RQ == 3 ? (nt ? linattn_prep_k<3, true> : linattn_prep_k<3, false>)
+                              : (nt ? linattn_prep_k<1, true> : linattn_prep_k<1, false>);
   // A launch has fewer than 2^32 threads: row groups beyond that (rows in the millions) go in further launches.
   const int64_t per = ((1LL << 32) - 1) / (64 * kLinRows * T);
   for (int64_t g0 = 0; g0 < groups; g0 += per) {

@@ -230,6 +230,35 @@ def test_linattn_prep_wide_rows(ext, dev):
             _ulp_close(o, r, nm, min_equal=0.98, steps=steps)
 
 
+@pytest.mark.parametrize("rep_qk,slots", [(False, 12900), (False, 12960), (True, 7300)])
+def test_linattn_prep_large_outputs(ext, dev, rep_qk, slots):
+    """Outputs on both sides of 256 MB (20768 or 37152 bytes a slot), from where the slot stores go past the caches:
+    every slot equals its row's values, which equal the oracle's; padding slots are zero."""
+    HV, HK = 48, 16
+    _say(f"case linattn_prep large slots={slots} rep_qk={rep_qk}")
+    LO, lay, proj, convw, A_log, dt_bias, KD, VD = _lin_inputs((6, [0], [0], [2]), HK, HV, seed=9, NB=1, PB=8)
+    N = lay["N"]
+    g = torch.Generator().manual_seed(slots)
+    row = torch.sort(torch.randint(0, N + 1, (slots,), generator=g)).values       # N = a padding slot
+    rep_ptr = torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(row, minlength=N + 1).cumsum(0)]).int()
+    rep_pos = torch.randperm(slots, generator=g).int()
+    d = lambda a: torch.as_tensor(a).to(dev).contiguous()  # noqa: E731
+    got = ext.linattn_prep_dedup2(proj.to(dev), d(lay["hist"]), d(rep_ptr), d(rep_pos), slots, convw.to(dev),
+                                  A_log.to(dev), dt_bias.to(dev), KD, VD, HV, HK, 128, rep_qk)
+    one = list(range(N + 1)) + [N + 1]                                             # one slot a row, one padding slot
+    want = LO.linattn_prep(proj, lay["hist"], one, list(range(N + 1)), N + 1, convw, A_log, dt_bias, KD, VD, HV, HK,
+                           128, rep_qk)
+    rowd, posd = row.to(dev), rep_pos.long().to(dev)
+    first = torch.tensor([int((row == n).nonzero()[0]) for n in range(N + 1)], device=dev)
+    for o, r, nm, steps in zip(got, want, "q k v g beta".split(), (2, 2, 1, 0, 1)):
+        by_row = o[posd]
+        assert torch.equal(by_row, by_row[first][rowd])
+        if nm == "g":
+            assert torch.allclose(by_row[first].cpu(), r, rtol=2e-6, atol=0)
+        else:
+            _ulp_close(by_row[first], r, nm, min_equal=0.98, steps=steps)
+
+
 def test_linattn_prep_more_rows_than_a_launch(ext, dev):
     """33.6 million packed rows of the smallest width: their row groups take two launches. Rows at both ends and around
     the cut hold one slot each (no history), the others none; the padding slots belong to the second launch."""
