@@ -346,8 +346,8 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const int epi, c
 namespace ojx {
 // The pick functions return a tile's kernel for an epilogue mode and weight layout, null where the tile has none; they
 // are instantiated beside the kernels. The persistent family has one kernel for each: a kernel that branches between
-// the bodies holds every body's scalars at once (256 x 256: 234 VGPRs and 47 spilled SGPRs with six bodies, 217-229
-// and none with one).
+// the bodies holds every body's scalars at once (256 x 256: 234 VGPRs and 47 spilled SGPRs with six bodies, 214-229
+// and none with one; seven of the other tiles spill 7-22 SGPRs, 256 x 288 with the residual 4-6 VGPRs too).
 typedef void (*GemmFn)(const GemmParams, const int epi);
 // Persistent stream-K family (gemm_sk.hip; instantiated there for the shapes of the tile table).
 template <int FN, int FM, int WN, int WM>

@@ -470,8 +470,10 @@ __global__ void __launch_bounds__(512) gemm_kx_kernel(const GemmParams p, const 
   else kx_dir<FW, FX, XE, XD, EPI_BF16>(p);
 }
 
-// One kernel for every epilogue and layout: unlike the persistent family's, it gains nothing from being split (the
-// 144 x 288 and 128 x 288 tiles spill 120-360 registers in kernels of one epilogue, none here).
+// One kernel for every epilogue and layout: unlike the persistent family's, it loses by being split (144 x 128 3-5%,
+// 144 x 288 up to 3% slower in kernels of one epilogue; 128 x 64 2.5% faster). The compiler gives the 144 x 288 and
+// 128 x 288 kernels 276 and 104 bytes of scratch a lane; in the assembly every access to it stands in the epilogues,
+// none among the MFMAs of the stage loop.
 template <int FW, int FX, int XE, int XD>
 GemmFn kx_pick(int epi, bool) {
   const bool prep = FW == 16 && XE == 0;  // the 256-row tiles also carry the full-attention prep epilogue
