@@ -1,8 +1,11 @@
-"""Runs one projection configuration repeatedly, for rocprofv3 (kernel traces and --pmc counter passes).
+"""Runs one projection configuration or performance case repeatedly, for rocprofv3 (kernel traces and --pmc counter
+passes).
 
     rocprofv3 --kernel-trace --stats -d /tmp/prof -- python3 open-jev-fast_amd/prof.py --shape gate_up --m 288
     rocprofv3 --pmc FETCH_SIZE -d /tmp/pmc -- python3 open-jev-fast_amd/prof.py --shape gate_up --m 288
     python3 open-jev-fast_amd/prof.py --copy-mb 512     # plain copy kernel, to calibrate FETCH_SIZE / WRITE_SIZE
+    python3 open-jev-fast_amd/prof.py --case linin_m384_rowmajor   # a case of perf/cases.py: a listed name, or a
+                                                                    # case as JSON; calls go over four sets of inputs
     (--packed: weights in the packed layout of ext.pack_weight, the layout bench.py uses by default; --zero-w:
     all-zero weights, to see how much of a kernel's time depends on the operands' values)
 
@@ -33,7 +36,20 @@ def main():
     ap.add_argument("--packed", action="store_true", help="weights in the packed layout (ext.pack_weight)")
     ap.add_argument("--zero-w", action="store_true", help="all-zero weights: the same data movement and MFMA "
                     "count with operands that draw less power (the clock's dependence on the data)")
+    ap.add_argument("--case", default="", help="a case of perf/cases.py: a listed name, or JSON")
     args = ap.parse_args()
+    if args.case:
+        import json
+        sys.path.insert(0, os.path.join(os.path.dirname(HERE), "perf"))
+        import cases
+        case = json.loads(args.case) if args.case.startswith("{") else {c["name"]: c for c in cases.listed()}[args.case]
+        states = [cases.prepare(case, seed) for seed in range(4)]
+        torch.cuda.synchronize()
+        for i in range(args.calls):
+            cases.run(states[i % len(states)])
+        torch.cuda.synchronize()
+        print(f"{case} calls={args.calls}", flush=True)
+        return
     if args.copy_mb:
         n = args.copy_mb << 20
         a = torch.ones(n // 4, dtype=torch.float32, device="cuda")
